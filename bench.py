@@ -202,8 +202,9 @@ def short_kernel(name):
     if m:
         f8 = m.group(4).strip(",").split(",")[0] if m.group(4) else "0"  # the FP8 flag: 0, or the A format + 1
         n = f"{m.group(1)}<{m.group(2)},{m.group(3)}>" + ("<f8>" if f8 not in ("0", "false") else "")
-    if n.startswith("gemm_wgrad_kernel<"):
-        n = "gemm_wgrad_kernel"
+    for one in ("gemm_wgrad_kernel", "router_fused_kernel"):  # one role whatever the template arguments
+        if n.startswith(one + "<"):
+            n = one
     # the persistent 256 x 256 kernels: B layout, epilogue and row gather (rows), row gather (weight gradient)
     m = re.match(r"g256::rows_kernel<(\d+),(\d+),(true|false)", n)
     if m:
@@ -219,8 +220,7 @@ def launch_roles(c):
     fs, f = c["fs"], c["f"]
     own = bool(fs) and fs != f  # shared expert of its own width: dense backward GEMMs on a helper stream
     r = {
-        "router_logits_kernel": ["router_topk"], "router_fused_kernel<64,2>": ["router_topk"],
-        "router_fused_kernel<128,4>": ["router_topk"], "router_fused_kernel<256,4>": ["router_topk"],
+        "router_logits_kernel": ["router_topk"], "router_fused_kernel": ["router_topk"],
         "router_select_lane_kernel<8>": ["router_select"],
         "router_select_lane_kernel<16>": ["router_select"], "router_select_kernel<1>": ["router_select"],
         "router_select_kernel<2>": ["router_select"], "router_select_kernel<4>": ["router_select"],
@@ -303,7 +303,7 @@ def label_launches(rows, c):
     out, seen = [], {}
     for row in sorted(rows, key=lambda x: int(x["Correlation_Id"])):
         k = short_kernel(row["Kernel_Name"])
-        if k == "router_logits_kernel" or k.startswith("router_fused_kernel"):
+        if k in ("router_logits_kernel", "router_fused_kernel"):
             seen = {}
         if g256 and fs and k in ("gemm_rows_kernel<1,1>", "gemm_rows_kernel<1,0>"):
             # with helper streams the shared expert's dense forward runs on the classic kernels beside the router,

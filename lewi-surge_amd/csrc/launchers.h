@@ -11,9 +11,9 @@ namespace lsurge {
 int router_topk_impl(const void* x, const void* w_r, const float* bias, int64_t t, int64_t d, int64_t e, int64_t k,
                      float* logits, int32_t* sel, float* weights, hipStream_t s, hipEvent_t after_logits,
                      int32_t* hist = nullptr);
-// Shapes the workgroup-fused router takes (logits, top-k, softmax and the per-64-token expert histograms in one
-// kernel): e in {32, 64, 128}, k <= 8, d a multiple of 64.  router_topk_impl uses it when given hist
-// ([ceil(t / 64)][e] int32, the layout's chunk counts for chunks of 64 tokens).
+// Shapes the fused router takes (logits, top-k, softmax and the per-64-token expert histograms in one
+// kernel): e in {32, 64, 128, 256}, k <= 8, d a multiple of 64.  router_topk_impl uses it when given hist
+// ([ceil(t / 64)][e] words, the layout's counts for chunks of 64 tokens: a count is the sum of its word's four bytes).
 bool router_fused_ok(int64_t d, int64_t e, int64_t k);
 
 // ---- routing layout (layout.hip)
@@ -42,7 +42,8 @@ struct LayoutTiles {
   ChunkTableOut chunks;
 };
 // Optional per-chunk expert histograms made by the caller (the fused router): hist [nchunk][E] for chunks of
-// waves x 64 consecutive slots (overwritten with the per-expert chunk bases); the layout then skips its own.
+// waves x 64 consecutive slots (a count is the sum of its word's four bytes; overwritten with the per-expert chunk
+// bases); the layout then skips its own.
 struct LayoutChunks {
   int32_t* hist = nullptr;
   int waves = 0;

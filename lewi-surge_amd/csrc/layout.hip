@@ -142,6 +142,11 @@ __device__ __forceinline__ void write_layout_tables(int E, const int32_t* gs_s, 
   }
 }
 
+// A count of the caller's histograms (LayoutChunks): the sum of the word's four bytes.  The layout's own are plain.
+__device__ __forceinline__ int hist_count(int v, bool packed) {
+  return packed ? (int)__builtin_amdgcn_sad_u8((uint32_t)v, 0u, 0u) : v;
+}
+
 // One workgroup of 1024 threads (at least E).  hist [nchunk][E] is overwritten with the exclusive per-expert
 // chunk base.
 // Thread (e, j) owns expert e's chunks [j cpt, (j + 1) cpt), kept in registers between the two passes (up to
@@ -149,7 +154,7 @@ __device__ __forceinline__ void write_layout_tables(int E, const int32_t* gs_s, 
 // markers of row_src are spread over all threads.  With tiles.t_expert set it also writes the 256-row tile table of
 // the layer's grouped GEMMs (see LayoutTiles), and with tiles.chunks.c_expert the weight gradients' chunk table.
 constexpr int LS_REG = 16, LS_BATCH = 32;
-__global__ __launch_bounds__(1024) void layout_scan_kernel(int32_t* __restrict__ hist, int nchunk, int E,
+__global__ __launch_bounds__(1024) void layout_scan_kernel(int32_t* __restrict__ hist, bool packed, int nchunk, int E,
                                                            int32_t* __restrict__ group_sizes,
                                                            int32_t* __restrict__ offsets,
                                                            int32_t* __restrict__ block_off,
@@ -172,7 +177,7 @@ __global__ __launch_bounds__(1024) void layout_scan_kernel(int32_t* __restrict__
     int sum = 0;
     if (in_regs) {
 #pragma unroll
-      for (int u = 0; u < LS_REG; ++u) v[u] = c0 + u < c1 ? hist[(int64_t)(c0 + u) * E + e_t] : 0;
+      for (int u = 0; u < LS_REG; ++u) v[u] = c0 + u < c1 ? hist_count(hist[(int64_t)(c0 + u) * E + e_t], packed) : 0;
 #pragma unroll
       for (int u = 0; u < LS_REG; ++u) sum += v[u];
     } else {  // LS_BATCH loads in flight per step: the scan is one round trip per batch, not per 8 chunks
@@ -181,7 +186,7 @@ __global__ __launch_bounds__(1024) void layout_scan_kernel(int32_t* __restrict__
 #pragma unroll
         for (int u = 0; u < LS_BATCH; ++u) wb[u] = c + u < c1 ? hist[(int64_t)(c + u) * E + e_t] : 0;
 #pragma unroll
-        for (int u = 0; u < LS_BATCH; ++u) sum += wb[u];
+        for (int u = 0; u < LS_BATCH; ++u) sum += hist_count(wb[u], packed);
       }
     }
     part_s[j_t * E + e_t] = sum;
@@ -213,7 +218,7 @@ __global__ __launch_bounds__(1024) void layout_scan_kernel(int32_t* __restrict__
 #pragma unroll
         for (int u = 0; u < LS_BATCH; ++u) {
           if (c + u < c1) hist[(int64_t)(c + u) * E + e_t] = run;
-          run += wb[u];
+          run += hist_count(wb[u], packed);
         }
       }
     }
@@ -372,8 +377,9 @@ __global__ __launch_bounds__(1024) void layout_fused_kernel(
       }
 #pragma unroll
       for (int u = 0; u < LF_LOADS; ++u) {
-        all += v[u];
-        below += c0 + u * tpe < me ? v[u] : 0;
+        const int n = hist_count(v[u], true);
+        all += n;
+        below += c0 + u * tpe < me ? n : 0;
       }
     }
     part[j_t * E + e_t] = below;
@@ -463,7 +469,7 @@ int layout_common(const int32_t* flat, int64_t M, int64_t E, int32_t* gs, int32_
   const unsigned scan_threads = 1024;
   if (M == 0) {
     LSURGE_LAUNCH(KID_LAYOUT_SCAN, s,
-                  hipLaunchKernelGGL(layout_scan_kernel, dim3(1), dim3(scan_threads), 0, s, hist, 0, (int)E, gs, offsets,
+                  hipLaunchKernelGGL(layout_scan_kernel, dim3(1), dim3(scan_threads), 0, s, hist, false, 0, (int)E, gs, offsets,
                                      block_off, row_src, blk_expert, blk_rows, num_blocks, (int)max_blocks, tiles));
     return LSURGE_OK;
   }
@@ -482,7 +488,7 @@ int layout_common(const int32_t* flat, int64_t M, int64_t E, int32_t* gs, int32_
                   hipLaunchKernelGGL(layout_hist_kernel, dim3((unsigned)nchunk), dim3(LT_THREADS),
                                      sizeof(int32_t) * LT_WAVES * (size_t)E, s, flat, M, (int)E, hist));
   LSURGE_LAUNCH(KID_LAYOUT_SCAN, s,
-                hipLaunchKernelGGL(layout_scan_kernel, dim3(1), dim3(scan_threads), 0, s, hist, (int)nchunk, (int)E, gs,
+                hipLaunchKernelGGL(layout_scan_kernel, dim3(1), dim3(scan_threads), 0, s, hist, pre.hist != nullptr, (int)nchunk, (int)E, gs,
                                    offsets, block_off, row_src, blk_expert, blk_rows, num_blocks,
                                    (int)max_blocks, tiles));
   LSURGE_LAUNCH(KID_LAYOUT_RANK, s,

@@ -464,10 +464,10 @@ static int moe_fwd_impl(const lsurge_moe_shape* s, const lsurge_moe_params* p, c
                  workspace_bytes);
   int32_t* rhist = hist_bytes ? (int32_t*)workspace : nullptr;
   // bf16: the shared expert's dense GEMMs fork at the start of the call and run on the classic kernels, whose
-  // workgroups (72 KiB of LDS, 4 waves) share a CU with the fused router's (66 KiB, 8 waves): MFMA-bound beside
-  // VALU-bound.  The persistent kernels take a CU's whole LDS, so beside them the router would wait for whole GEMMs.
-  // C2: 1.547 -> 1.537 ms per step, forward 0.537 -> 0.528 ms (same-box A/B against forking after the router with
-  // the persistent kernels).
+  // workgroups (72 KiB of LDS, 4 waves) share a CU with the fused router's (9 KiB, 2 waves at 64 experts), whose f32
+  // matrix steps leave the memory path free.  The persistent kernels take a CU's whole LDS, so beside them the router would wait for whole GEMMs.
+  // C2, measured with the vector-unit router before this one: 1.547 -> 1.537 ms per step (same-box A/B against forking
+  // after the router with the persistent kernels).
   const bool early = !w8 && q.fs && s0 != st;
   // a merged shared expert forked early: its down projection rides along the routed down GEMM as expert E (its
   // tiles follow the routed ones in the tile table), so the helper's classic-kernel GEMMs end with the layout

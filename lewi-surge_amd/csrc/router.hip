@@ -8,8 +8,8 @@
 // Two paths.  The split path (the ABI's lsurge_router_topk, and shapes the fused kernel does not take): a logits
 // kernel over (token block, expert block) tiles, then a selection kernel (one lane per token from 8192 tokens, else
 // one wave per token).  The layer's fused path (E = 32, 64, 128 or 256, k <= 8): router_fused_kernel, one workgroup
-// of 64 tokens x all experts computing the same logits, then top-k, softmax and the layout's per-64-token expert
-// histograms in the same workgroup (described at the kernel).
+// of 16 to 64 tokens x all experts computing the same logits on the f32 matrix cores, then top-k, softmax and the
+// layout's per-64-token expert histograms in the same workgroup (described at the kernel).
 #include "launchers.h"
 
 
@@ -284,131 +284,146 @@ __global__ __launch_bounds__(RL_THREADS) void router_logits_kernel(const bf16_t*
 }
 
 // ---------------------------------------------------------------------------------------------- workgroup-fused path
-// Fused router of the layer (E = 32, 64, 128 or 256 experts, k <= 8): one workgroup = 64 tokens x all EP experts (EP =
-// E rounded up to a multiple of 64; the padding experts get zero weights and are never selected).  Each thread
-// accumulates 4 tokens x EL experts (EL = 2 or 4): per d step one f32x4 LDS read of x (its 4 tokens, the same address
-// for the 16 lanes of its row) and one EL-wide read of w, then 4 EL FMAs.  Wave w covers the token quads 4 (w % 4) ..
-// + 3 (one per row of 16 lanes) and the experts 16 EL (w / 4) ..  The sum over d is the sequential f32 fmaf chain of
-// the split path, so the logits are bitwise those of router_logits_kernel.  Then, in the same workgroup:
-//  - the logits go to HBM and to an LDS tile [64][EP + 1];
-//  - top-k + softmax per token: L = EP / (4 EL) lanes per token each keep a sorted list of the best 8 of their
-//    EPL = 4 EL experts (scanned in ascending expert order, a logit moves ahead only of strictly smaller ones), and
+// Fused router of the layer (E = 32, 64, 128 or 256 experts, k <= 8): logits on the f32 matrix cores, then top-k,
+// softmax and the expert histogram in the same workgroup.
+//
+// Logits.  v_mfma_f32_16x16x4_f32 adds its four products to the accumulator one after the other in ascending k, each
+// with one f32 rounding: exactly the fmaf chain of router_logits_kernel, at twice the vector unit's rate (measured
+// bit-equal on normal, wide-range, cancelling, subnormal and non-finite bf16 operands; the GPU tests compare the two
+// kernels bit for bit).  One workgroup = TOK = 16 TT tokens x all E experts, one wave per 32 experts; a wave holds TT
+// token tiles x 2 expert tiles (expert 32 wave + 2 c + h is column c of tile h, so one dword of a row of W_r feeds
+// both tiles).  Step s of a 32-deep block covers d = 4 s .. + 3, lane quarter q supplying d = 4 s + q:
+//   x  goes through a double LDS buffer of DC-deep chunks, each block of a row stored by quarter ([q][8 steps] bf16),
+//      so one 16-byte read gives a lane its operands of 8 steps; blocks are read one ahead of their use;
+//   w  straight from L2 into registers, a ring of GD / 4 steps ahead of its use.
+// Bound by the matrix pipe (64 cycles a step and token tile) once two waves share a SIMD, by load latency below that.
+// TT = 1 gives the most workgroups, TT = 4 the fewest reads of W_r; the launcher takes the largest TT that still
+// leaves 2048 waves (two per SIMD), so small batches spread over the CUs and a 1 MB W_r is read once per 64 tokens.
+// At E = 256 the registers are held to 128, so that two 8-wave workgroups share a CU (656 -> 613 us at T = 65536, d =
+// 2048); elsewhere the bound cost more than it gave.
+// Replaced a vector-FMA kernel (4 tokens x 2-4 experts a thread, both operands as f32 through LDS, whose bandwidth
+// bounded it).  Alone, before -> after: T = 4096, E = 64, d = 1024 45 -> 20 us; T = 16384, E = 64 55 -> 31 us; T =
+// 16384, E = 128 97 -> 49 us; T = 65536, E = 256, d = 2048 1088 -> 613 us (matrix pipe alone: 455 us at the 150
+// TFLOP/s that this instruction reaches).
+//
+// Then, in the same workgroup:
+//  - the logits go to HBM and to an LDS tile [TOK][E + 1];
+//  - top-k + softmax per token: L = E / (8 TT) lanes per token each keep a sorted list of the best 8 of their
+//    EPL = 8 TT experts (scanned in ascending expert order, a logit moves ahead only of strictly smaller ones), and
 //    k merge rounds take the best head of the L lists (larger logit, ties to the lower expert index) -- the order of
 //    a stable descending sort, as in router_select_lane_kernel, whose softmax (in rank order) this repeats;
-//  - the expert histogram of the workgroup's 64 k slots (LDS counters) -> hist[blockIdx.x][E], the layout's
-//    per-chunk counts (chunks of 64 tokens).
-// This replaces the selection kernel, the layout's histogram kernel and the logits round trip between them.
-// LDS: double-buffered x [DC][64] and w [DC][EP] f32 chunks (DC = 32 at EP = 256, else 64); after the d loop the
-// same bytes hold the logits tile.
-constexpr int RF_TOK = 64, RF_XP = RF_TOK + 4;
-
-template <int EP, int EL>
-__global__ __launch_bounds__(16 * EP / EL) void router_fused_kernel(const bf16_t* __restrict__ x,
-                                                                    const bf16_t* __restrict__ w,
-                                                                    const float* __restrict__ bias, int T, int d,
-                                                                    int E, int k, float* __restrict__ logits,
-                                                                    int32_t* __restrict__ sel,
-                                                                    float* __restrict__ weights,
-                                                                    int32_t* __restrict__ hist) {
-  constexpr int NT = 16 * EP / EL, L = NT / RF_TOK, EPL = EP / L;  // threads, lanes per token, experts per lane
-  constexpr int DC = EP >= 256 ? 32 : 64;
-  static_assert(EP % 64 == 0 && (EL == 2 || EL == 4) && EPL == 4 * EL && 64 % L == 0, "fused router shape");
-  constexpr int XS_EL = 2 * DC * RF_XP, WS_EL = 2 * DC * EP, TILE_EL = RF_TOK * (EP + 1);
-  constexpr int SM_EL = XS_EL + WS_EL > TILE_EL ? XS_EL + WS_EL : TILE_EL;
-  __shared__ __attribute__((aligned(16))) float sm[SM_EL];
-  __shared__ int32_t cnt[EP];
-  float(*xs)[DC][RF_XP] = reinterpret_cast<float(*)[DC][RF_XP]>(sm);
-  float(*ws)[DC][EP] = reinterpret_cast<float(*)[DC][EP]>(sm + XS_EL);
+//  - the expert histogram of the workgroup's TOK k slots (LDS counters) -> hist[chunk of 64 tokens][E], the layout's
+//    per-chunk counts.  A word of hist holds the counts of its chunk's four 16-token quarters in its bytes (a token
+//    picks an expert at most once, so even 64 tokens fit one byte): a workgroup writes the TT bytes of its own
+//    quarters (its count and zeros), and the layout adds the four bytes up.  No workgroup touches another's bytes, so
+//    nothing has to be cleared first.
+template <int E, int TT, int DC>
+__global__ __launch_bounds__(2 * E, E == 256 ? 4 : 1) void router_fused_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+                                                             const float* __restrict__ bias, int T, int d, int k,
+                                                             float* __restrict__ logits, int32_t* __restrict__ sel,
+                                                             float* __restrict__ weights, uint8_t* __restrict__ hist) {
+  constexpr int NT = 2 * E, TOK = 16 * TT, L = NT / TOK, EPL = E / L;  // threads, tokens, lanes and experts a lane
+  constexpr int GD = DC < 128 ? DC : 128;    // depth of the weight ring
+  constexpr int XP = 2 * DC + 16;            // LDS row pitch in bytes (rows one 16-byte slot apart in the banks)
+  static_assert(64 % L == 0 && L >= 1 && EPL >= 8, "fused router shape");
+  constexpr int XS_B = 2 * TOK * XP, TILE_B = TOK * (E + 1) * 4;
+  __shared__ __attribute__((aligned(16))) char sm[XS_B > TILE_B ? XS_B : TILE_B];
+  __shared__ int32_t cnt[E];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int t0 = blockIdx.x * RF_TOK;
-  const int tq = 4 * (wv & 3) + (lane >> 4);    // token quad (tokens t0 + 4 tq ..)
-  const int eq = 16 * (wv >> 2) + (lane & 15);  // experts EL eq .. EL eq + EL - 1
-  float acc[4][EL];
+  const int t0 = blockIdx.x * TOK;
+  const int r = lane & 15, q = lane >> 4;
+  for (int e = tid; e < E; e += NT) cnt[e] = 0;
+  // staging: x pieces p = tid + NT i: token p / (DC / 8), d 8 (p % (DC / 8)) .. + 7 of the chunk (zeros past T), which
+  // are two steps of every quarter
+  constexpr int XQ = TOK * (DC / 8), XR = (XQ + NT - 1) / NT;
+  u32x4 xr[XR];
+  auto gx = [&](int d0) {
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int j = 0; j < EL; ++j) acc[a][j] = 0.f;
-  for (int e = tid; e < EP; e += NT) cnt[e] = 0;
-  // staging: x pieces q = tid + NT r (q < XQ): token q % 64, d offset 8 (q / 64); w pieces p = tid + NT r: d row
-  // p / (EP / 8), experts 8 (p % (EP / 8)) .. (zeros past E)
-  constexpr int XQ = RF_TOK * (DC / 8), XR = (XQ + NT - 1) / NT, WQ = DC * EP / 8, WR = WQ / NT;
-  static_assert(WR * NT == WQ, "w pieces split evenly over the threads");
-  const int xtt = tid & 63;
-  u32x4 xr[XR], wr[WR];
-  auto gload = [&](int d0) {
-    const int t = t0 + xtt;
-#pragma unroll
-    for (int r = 0; r < XR; ++r) {
-      const int q = tid + NT * r;
-      if (q < XQ) xr[r] = t < T ? *reinterpret_cast<const u32x4*>(x + (int64_t)t * d + d0 + 8 * (q >> 6)) : u32x4{0, 0, 0, 0};
-    }
-#pragma unroll
-    for (int r = 0; r < WR; ++r) {
-      const int p = tid + NT * r, row = p / (EP / 8), e8 = 8 * (p % (EP / 8));
-      wr[r] = e8 < E ? *reinterpret_cast<const u32x4*>(w + (int64_t)(d0 + row) * E + e8) : u32x4{0, 0, 0, 0};
+    for (int i = 0; i < XR; ++i) {
+      const int p = tid + NT * i, t = t0 + p / (DC / 8);
+      xr[i] = p < XQ && t < T ? *reinterpret_cast<const u32x4*>(x + (int64_t)t * d + d0 + 8 * (p % (DC / 8)))
+                              : u32x4{0, 0, 0, 0};
     }
   };
-  auto sstore = [&](int buf) {
-    float v[8];
+  auto sx = [&](int buf) {
 #pragma unroll
-    for (int r = 0; r < XR; ++r) {
-      const int q = tid + NT * r;
-      if (q < XQ) {
-        unpack_bf16x8(xr[r], v);
+    for (int i = 0; i < XR; ++i) {
+      const int p = tid + NT * i, c = p % (DC / 8);
+      if (p < XQ) {
+        char* o = sm + buf * TOK * XP + (p / (DC / 8)) * XP + 64 * (c >> 2) + 4 * (c & 3);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) xs[buf][8 * (q >> 6) + i][xtt] = v[i];
+        for (int h = 0; h < 2; ++h) {  // quarters 2 h and 2 h + 1: elements (q, q + 4) of the piece
+          *reinterpret_cast<uint32_t*>(o + 32 * h) = __builtin_amdgcn_perm(xr[i][2 + h], xr[i][h], 0x05040100u);
+          *reinterpret_cast<uint32_t*>(o + 32 * h + 16) = __builtin_amdgcn_perm(xr[i][2 + h], xr[i][h], 0x07060302u);
+        }
       }
     }
-#pragma unroll
-    for (int r = 0; r < WR; ++r) {
-      const int p = tid + NT * r, row = p / (EP / 8), e8 = 8 * (p % (EP / 8));
-      unpack_bf16x8(wr[r], v);
-      *reinterpret_cast<f32x4*>(&ws[buf][row][e8]) = f32x4{v[0], v[1], v[2], v[3]};
-      *reinterpret_cast<f32x4*>(&ws[buf][row][e8 + 4]) = f32x4{v[4], v[5], v[6], v[7]};
-    }
   };
-  gload(0);
+  const bf16_t* wl = w + (int64_t)q * E + 32 * wv + 2 * r;  // this lane's experts of d row q
+  auto gw = [&](int dd) { return *reinterpret_cast<const uint32_t*>(wl + (int64_t)dd * E); };
+  f32x4 acc[TT][2];
+#pragma unroll
+  for (int a = 0; a < TT; ++a) acc[a][0] = acc[a][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  uint32_t wr[GD / 4];
+  gx(0);
+#pragma unroll
+  for (int s = 0; s < GD / 4; ++s) wr[s] = gw(4 * s);
+  u32x4 fa[2][TT];
   int buf = 0;
-  for (int d0 = 0; d0 < d; d0 += DC, buf ^= 1) {  // d % 64 == 0 (checked on the host)
-    sstore(buf);
+  for (int d0 = 0; d0 < d; d0 += DC, buf ^= 1) {  // d % DC == 0 (checked on the host)
+    // buffer buf was last read two chunks ago, before the barrier of the previous chunk
+    sx(buf);
     __syncthreads();
-    if (d0 + DC < d) gload(d0 + DC);
-#pragma unroll 8
-    for (int dd = 0; dd < DC; ++dd) {
-      const f32x4 xv = *reinterpret_cast<const f32x4*>(&xs[buf][dd][4 * tq]);
-      float wv[EL];
-      if constexpr (EL == 4) {
-        const f32x4 w4 = *reinterpret_cast<const f32x4*>(&ws[buf][dd][4 * eq]);
+    gx(min(d0 + DC, d - DC));  // the next chunk (the last one again at the end, unused)
+    const char* xa = sm + buf * TOK * XP + r * XP + 16 * q;  // this lane's row and quarter
+    auto fread = [&](u32x4(&f)[TT], int blk) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) wv[j] = w4[j];
-      } else {
-        typedef float f32x2 __attribute__((ext_vector_type(2)));
-        const f32x2 w2 = *reinterpret_cast<const f32x2*>(&ws[buf][dd][2 * eq]);
-        wv[0] = w2[0];
-        wv[1] = w2[1];
+      for (int a = 0; a < TT; ++a) f[a] = *reinterpret_cast<const u32x4*>(xa + 16 * a * XP + 64 * blk);
+    };
+    fread(fa[0], 0);
+    for (int g = 0; g < DC; g += GD) {
+      const int dn = min(d0 + g + GD, d - GD);  // the ring's next depth (the last one again at the end, unused)
+#pragma unroll
+      for (int b = 0; b < GD / 32; ++b) {
+        fread(fa[(b + 1) & 1], min(g / 32 + b + 1, DC / 32 - 1));
+        float wc[8][2];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+          wc[s][0] = __uint_as_float(wr[8 * b + s] << 16);
+          wc[s][1] = __uint_as_float(wr[8 * b + s] & 0xffff0000u);
+          wr[8 * b + s] = gw(dn + 32 * b + 4 * s);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+#pragma unroll
+          for (int a = 0; a < TT; ++a) {
+            const uint32_t u = fa[b & 1][a][s >> 1];
+            const float xv = __uint_as_float(s & 1 ? u & 0xffff0000u : u << 16);
+            acc[a][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv, wc[s][0], acc[a][0], 0, 0, 0);
+            acc[a][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv, wc[s][1], acc[a][1], 0, 0, 0);
+          }
+        __builtin_amdgcn_sched_barrier(0);
       }
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int j = 0; j < EL; ++j) acc[a][j] = __builtin_fmaf(xv[a], wv[j], acc[a][j]);
     }
   }
   __syncthreads();  // every wave is done with the staging buffers: they now hold the logits tile
-  float* lt = sm;
+  float* lt = reinterpret_cast<float*>(sm);
+  const int e0 = 32 * wv + 2 * r;
+  const float b0 = bias ? bias[e0] : 0.f, b1 = bias ? bias[e0 + 1] : 0.f;
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    const int tt = 4 * tq + a, t = t0 + tt;
+  for (int a = 0; a < TT; ++a)
 #pragma unroll
-    for (int j = 0; j < EL; ++j) {
-      const int e = EL * eq + j;
-      const float v = bias && e < E ? acc[a][j] + bias[e] : acc[a][j];
-      lt[tt * (EP + 1) + e] = v;
-      if (t < T && e < E) logits[(int64_t)t * E + e] = v;
+    for (int i = 0; i < 4; ++i) {  // accumulator element i: token 4 q + i of the tile
+      const int tt = 16 * a + 4 * q + i, t = t0 + tt;
+      const float v0 = bias ? acc[a][0][i] + b0 : acc[a][0][i], v1 = bias ? acc[a][1][i] + b1 : acc[a][1][i];
+      lt[tt * (E + 1) + e0] = v0;
+      lt[tt * (E + 1) + e0 + 1] = v1;
+      if (t < T) *reinterpret_cast<float2*>(logits + (int64_t)t * E + e0) = float2{v0, v1};
     }
-  }
   __syncthreads();
-  // selection: token tid / L, lane part tid % L scans experts part, part + L, ... (ascending, below E) into a sorted
-  // list of its best KL = 8 (k <= 8, so a lane's share of the top k is always in it; the rest never matter)
+  // selection: token tid / L, lane part tid % L scans experts part, part + L, ... (ascending) into a sorted list of
+  // its best KL = 8 (k <= 8, so a lane's share of the top k is always in it; the rest never matter)
   constexpr int KL = 8;
   const int tt = tid / L, part = tid % L, t = t0 + tt;
   float tv[KL];
@@ -421,13 +436,12 @@ __global__ __launch_bounds__(16 * EP / EL) void router_fused_kernel(const bf16_t
 #pragma unroll 1
   for (int c = 0; c < EPL; ++c) {
     const int e = part + L * c;
-    const bool valid = e < E;  // padding experts are never inserted
-    float cv = lt[tt * (EP + 1) + e];
+    float cv = lt[tt * (E + 1) + e];
     int ci = e;
     bool placed = false;
 #pragma unroll
     for (int j = 0; j < KL; ++j) {
-      const bool g = valid && (placed || ti[j] < 0 || cv > tv[j]);
+      const bool g = placed || ti[j] < 0 || cv > tv[j];
       const float ov = tv[j];
       const int oi = ti[j];
       tv[j] = g ? cv : ov;
@@ -483,7 +497,14 @@ __global__ __launch_bounds__(16 * EP / EL) void router_fused_kernel(const bf16_t
     }
   }
   __syncthreads();
-  for (int e = tid; e < E; e += NT) hist[(int64_t)blockIdx.x * E + e] = cnt[e];
+  // this workgroup's quarters of the 64-token chunk's words
+  constexpr int PER = 4 / TT;
+  uint8_t* hq = hist + (int64_t)(blockIdx.x / PER) * E * 4 + (blockIdx.x % PER) * TT;
+  for (int e = tid; e < E; e += NT) {
+    if constexpr (TT == 1) hq[4 * e] = (uint8_t)cnt[e];
+    else if constexpr (TT == 2) *reinterpret_cast<uint16_t*>(hq + 4 * e) = (uint16_t)cnt[e];
+    else *reinterpret_cast<uint32_t*>(hq + 4 * e) = (uint32_t)cnt[e];
+  }
 }
 
 // one wave per token: top-k (larger logit first, ties to the lower expert index), softmax over the k
@@ -618,16 +639,35 @@ int lsurge::router_topk_impl(const void* x, const void* w_r, const float* bias, 
   if (hist) {  // workgroup-fused path: logits, top-k, softmax and the per-64-token histograms in one kernel
     LSURGE_REQUIRE(logits && router_fused_ok(d, e, k), "router_topk: shape d=%lld e=%lld k=%lld has no fused kernel",
                    (long long)d, (long long)e, (long long)k);
-    const dim3 grid((unsigned)((t + RF_TOK - 1) / RF_TOK));
-#define RF_CASE(EP, EL)                                                                                          \
-  LSURGE_LAUNCH(KID_ROUTER, s,                                                                                   \
-                hipLaunchKernelGGL((router_fused_kernel<EP, EL>), grid, dim3(16 * EP / EL), 0, s, (const bf16_t*)x, \
-                                   (const bf16_t*)w_r, bias, (int)t, (int)d, (int)e, (int)k, logits, sel, weights, \
-                                   hist))
-    if (e <= 64) RF_CASE(64, 2);
-    else if (e == 128) RF_CASE(128, 4);
-    else RF_CASE(256, 4);
+    // token tiles per wave: the largest of 4, 2, 1 that leaves two waves per SIMD (2048).  Measured alone, at 1 / 2 /
+    // 4: T = 4096, E = 64 20 / - / 55 us; T = 16384, E = 64 30 / 32 / 57; T = 16384, E = 128 53 / 49 / 80; T = 65536,
+    // E = 256, d = 2048 700 / 629 / 613
+    const int64_t chunks = (t + 63) / 64, per16 = chunks * 4 * (e / 32);  // waves at one tile each
+    const int tt = per16 / 4 >= 2048 ? 4 : per16 / 2 >= 2048 ? 2 : 1;
+    const dim3 grid((unsigned)(chunks * (4 / tt)));  // whole chunks: every byte of hist is written
+#define RF_LAUNCH(E_, TT_, DC_)                                                                                    \
+  LSURGE_LAUNCH(KID_ROUTER, s,                                                                                     \
+                hipLaunchKernelGGL((router_fused_kernel<E_, TT_, DC_>), grid, dim3(2 * E_), 0, s, (const bf16_t*)x, \
+                                   (const bf16_t*)w_r, bias, (int)t, (int)d, (int)k, logits, sel, weights,         \
+                                   (uint8_t*)hist))
+#define RF_DC(E_, TT_)                          \
+  do {                                          \
+    if (d % 128 == 0) RF_LAUNCH(E_, TT_, 128);  \
+    else RF_LAUNCH(E_, TT_, 64);                \
+  } while (0)
+#define RF_CASE(E_)                 \
+  do {                              \
+    if (tt == 4) RF_DC(E_, 4);      \
+    else if (tt == 2) RF_DC(E_, 2); \
+    else RF_DC(E_, 1);              \
+  } while (0)
+    if (e == 32) RF_CASE(32);
+    else if (e == 64) RF_CASE(64);
+    else if (e == 128) RF_CASE(128);
+    else RF_CASE(256);
 #undef RF_CASE
+#undef RF_DC
+#undef RF_LAUNCH
     if (after_logits && hipEventRecord(after_logits, s) != hipSuccess)
       return lsurge::set_error(LSURGE_ERR_LAUNCH, "router_topk: hipEventRecord failed");
     return LSURGE_OK;

@@ -118,6 +118,37 @@ def test_fused_router_ties(E, k, T, dev):
         assert np.array_equal(v[n], lay[n]), n
 
 
+@pytest.mark.parametrize("T,d,E,k", [(1, 64, 32, 1), (15, 192, 64, 6), (17, 128, 128, 8), (65, 64, 256, 8),
+                                     (129, 320, 64, 4), (8200, 64, 256, 8), (16400, 128, 256, 6), (16333, 64, 128, 6),
+                                     (32700, 64, 32, 4), (131072, 64, 32, 2)])
+def test_fused_router_matrix_core_chain(T, d, E, k, dev):
+    """The fused router's logits come from f32 matrix-core steps, the split router's from fmaf on the vector unit: the
+    same bits on every tile count per wave (1, 2, 4, chosen by T and E), both chunk depths, partial 64-token chunks,
+    and operands whose products cancel, fall below the normal range or are infinite; and the layout they lead to."""
+    from test_router_layout_gpu import gpu_router
+    rng = np.random.default_rng(T + E)
+    p = mo.make_inputs(T=T, d=d, E=E, k=k, f=64, fs=0, seed=E + k)
+    x, w_r = p["x"], p["w_r"]
+    x[0::4] *= np.float32(2.0 ** -64)
+    w_r[:, 1::8] *= np.float32(2.0 ** -60)       # with the rows above: products around 2^-130
+    x[1::4, 1::2] = -x[1::4, 0::2]               # pairs that almost cancel against near-equal columns
+    w_r[1::2, 2::8] = w_r[0::2, 2::8] * np.float32(1.0078125)
+    if T > 40:
+        x[40, 5] = np.inf                        # +-inf logits (w_r is never 0 there)
+    p["w_r"] = mo.round_bf16(w_r)
+    p["bias"] = None if T % 2 else rng.standard_normal(E).astype(np.float32)
+    layer = MoELayer(MoEShape(T, d, E, k, 64, 0), dev)
+    layer.forward(to_dev(p, dev))
+    v = {n: t.cpu().numpy() for n, t in layer.views().items() if t.dtype != torch.bfloat16}
+    logits_s, sel_s, wts_s = gpu_router(p["x"], p["w_r"], k, p["bias"], dev)
+    assert np.array_equal(v["logits"].view(np.uint32), logits_s.view(np.uint32))
+    assert np.array_equal(v["sel"], sel_s)
+    assert np.array_equal(v["weights"], wts_s, equal_nan=True)
+    lay = co.build_layout(sel_s, E)
+    for n in ("group_sizes", "offsets", "block_off", "order", "pos", "slot"):
+        assert np.array_equal(v[n], lay[n]), n
+
+
 def test_hot_experts_chunked_wgrad(dev):
     """Every token routes to experts 0 and 1 (a large bias), so each holds 5000 rows: the routed weight gradients
     cut them into 4096 + 904-row chunks summed from partials, and the six empty experts get zero gradients."""
