@@ -178,6 +178,12 @@ size_t lsurge_ragged_dot_bwd_f32_workspace_bytes(int64_t m, int64_t kdim, int64_
 int lsurge_ragged_dot_bwd(const void* lhs, const void* rhs, const int32_t* group_sizes, const void* g,
                           int64_t m, int64_t kdim, int64_t n, int64_t e, int in_dtype, void* dlhs, float* drhs,
                           void* workspace, size_t workspace_bytes, lsurge_stream_t stream);
+/* lsurge_ragged_dot_bwd with drhs [e, kdim, n] of drhs_dtype: LSURGE_F32, or in_dtype (the f32 result rounded once, to
+ * nearest even), which is what the reference's VJP returns (the einsum's operand gradients come back in their dtype,
+ * modal/padded_gmm.py:67-68), without an f32 copy of the gradient in between. */
+int lsurge_ragged_dot_bwd_as(const void* lhs, const void* rhs, const int32_t* group_sizes, const void* g,
+                             int64_t m, int64_t kdim, int64_t n, int64_t e, int in_dtype, void* dlhs, void* drhs,
+                             int drhs_dtype, void* workspace, size_t workspace_bytes, lsurge_stream_t stream);
 
 /* ------------------------------------------------------------------------------------------------
  * Whole MoE layer: router -> layout -> dispatch -> gate/up GEMM (+SiLU*mul) -> down GEMM -> combine
@@ -233,6 +239,12 @@ int lsurge_moe_fwd(const lsurge_moe_shape* s, const lsurge_moe_params* p, void* 
 /* dy: [t, d] bf16 upstream gradient.  `saved` must come from lsurge_moe_fwd with the same s and p. */
 int lsurge_moe_bwd(const lsurge_moe_shape* s, const lsurge_moe_params* p, const void* dy, const void* saved,
                    const lsurge_moe_grads* g, void* workspace, size_t workspace_bytes, lsurge_stream_t stream);
+/* lsurge_moe_bwd with the weight gradients (dw_r, dw_gate, dw_up, dw_down and the shared expert's) in dw_dtype:
+ * LSURGE_F32, or LSURGE_BF16 (each f32 gradient rounded once, to nearest even; those pointers of g then point at bf16
+ * values).  dx stays bf16 and dweights f32. */
+int lsurge_moe_bwd_as(const lsurge_moe_shape* s, const lsurge_moe_params* p, const void* dy, const void* saved,
+                      const lsurge_moe_grads* g, int dw_dtype, void* workspace, size_t workspace_bytes,
+                      lsurge_stream_t stream);
 
 /* Views into `saved` (device pointers), for tests and the Python surface. */
 typedef struct {

@@ -70,6 +70,7 @@ _SIGS = {
     "lsurge_ragged_dot_noalloc_max_groups": (_sz, []),
     "lsurge_ragged_dot_noalloc": (_int, [_p, _p, _p, _i64, _i64, _i64, _i64, _int, _p, _int, _p]),
     "lsurge_ragged_dot_bwd": (_int, [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _int, _p, _p, _p, _sz, _p]),
+    "lsurge_ragged_dot_bwd_as": (_int, [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _int, _p, _p, _int, _p, _sz, _p]),
     "lsurge_ragged_dot_bwd_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64]),
     "lsurge_moe_saved_bytes": (_sz, [ctypes.POINTER(MoeShape)]),
     "lsurge_moe_saved_bytes_fp8": (_sz, [ctypes.POINTER(MoeShape)]),
@@ -78,6 +79,8 @@ _SIGS = {
     "lsurge_moe_fwd": (_int, [ctypes.POINTER(MoeShape), ctypes.POINTER(MoeParams), _p, _p, _sz, _p, _sz, _p]),
     "lsurge_moe_bwd": (_int, [ctypes.POINTER(MoeShape), ctypes.POINTER(MoeParams), _p, _p, ctypes.POINTER(MoeGrads),
                               _p, _sz, _p]),
+    "lsurge_moe_bwd_as": (_int, [ctypes.POINTER(MoeShape), ctypes.POINTER(MoeParams), _p, _p, ctypes.POINTER(MoeGrads),
+                                 _int, _p, _sz, _p]),
     "lsurge_moe_saved_layout": (_int, [ctypes.POINTER(MoeShape), _p, ctypes.POINTER(MoeSavedViews)]),
     "lsurge_fp8_quantize_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "lsurge_fp8_quantize": (_int, [_p, _i64, _i64, _i64, _int, _p, _p, _p, _sz, _p]),

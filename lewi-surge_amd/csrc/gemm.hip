@@ -27,7 +27,7 @@ using CfgPP = GemmCfg<256, 256, 32, 2, 4, 3, 1, 1>;
 template <int V>
 __global__ void splitk_reduce_kernel(const float* __restrict__ part, int S, int E, int64_t I, int64_t N,
                                      float* __restrict__ C, float* __restrict__ C2, int64_t n_split, int64_t ldc,
-                                     int64_t c_estride) {
+                                     int64_t c_estride, int c_type) {
   typedef float fv __attribute__((ext_vector_type(V)));
   const int64_t total = (int64_t)E * I * N;
   for (int64_t x = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * V; x < total;
@@ -47,14 +47,19 @@ __global__ void splitk_reduce_kernel(const float* __restrict__ part, int S, int 
     for (; s < S; ++s) v += *reinterpret_cast<const fv*>(part + (int64_t)s * total + x);
     const int64_t e = x / (I * N), rem = x % (I * N);
     const int64_t row = rem / N, col = rem % N;
-    float* dst = (C2 && col >= n_split) ? C2 + e * c_estride + row * ldc + (col - n_split)
-                                        : C + e * c_estride + row * ldc + col;
-    *reinterpret_cast<fv*>(dst) = v;
+    const bool second = C2 && col >= n_split;
+    const int64_t o = e * c_estride + row * ldc + (second ? col - n_split : col);
+    float* dst = second ? C2 : C;
+    if constexpr (V == 4) store_grad4(dst, c_type, o, v);
+    else if (c_type == LSURGE_BF16) reinterpret_cast<bf16_t*>(dst)[o] = f32_to_bf16(v[0]);
+    else if (c_type == LSURGE_F16) reinterpret_cast<uint16_t*>(dst)[o] = f32_to_f16(v[0]);
+    else dst[o] = v[0];
   }
 }
 
 static int launch_splitk_reduce(const float* part, int S, int E, int64_t I, int64_t N, float* C, float* C2,
-                                int64_t n_split, int64_t ldc, int64_t c_estride, hipStream_t s) {
+                                int64_t n_split, int64_t ldc, int64_t c_estride, hipStream_t s,
+                                int c_type = LSURGE_F32) {
   const int64_t total = (int64_t)E * I * N;
   const bool v4 = N % 4 == 0 && n_split % 4 == 0 && ldc % 4 == 0 && c_estride % 4 == 0 &&
                   ((uintptr_t)C | (uintptr_t)C2 | (uintptr_t)part) % 16 == 0;
@@ -63,11 +68,11 @@ static int launch_splitk_reduce(const float* part, int S, int E, int64_t I, int6
   if (v4)
     LSURGE_LAUNCH(KID_SPLITK_REDUCE, s,
                   hipLaunchKernelGGL(splitk_reduce_kernel<4>, dim3(grid), dim3(256), 0, s, part, S, E, I, N, C, C2,
-                                     n_split, ldc, c_estride));
+                                     n_split, ldc, c_estride, c_type));
   else
     LSURGE_LAUNCH(KID_SPLITK_REDUCE, s,
                   hipLaunchKernelGGL(splitk_reduce_kernel<1>, dim3(grid), dim3(256), 0, s, part, S, E, I, N, C, C2,
-                                     n_split, ldc, c_estride));
+                                     n_split, ldc, c_estride, c_type));
   return LSURGE_OK;
 }
 
@@ -288,13 +293,13 @@ __global__ __launch_bounds__(WC_THREADS) void wgrad_chunks_kernel(const int32_t*
 }
 
 // dW of each split expert = its chunk partials summed in chunk order (f32, deterministic), -> C (and C2 for
-// columns >= n_split).  Grid-stride over (split expert, 4-element group).
+// columns >= n_split) in c_type.  Grid-stride over (split expert, 4-element group).
 __global__ void wgrad_chunk_reduce_kernel(const float* __restrict__ part, const int32_t* __restrict__ split_list,
                                           const int32_t* __restrict__ num_split, const int32_t* __restrict__ e_pbase,
                                           const int32_t* __restrict__ e_nparts, int64_t I, int64_t N,
                                           float* __restrict__ C, float* __restrict__ C2, int64_t n_split, int64_t ldc,
                                           int64_t c_estride, int x_expert, float* __restrict__ Cx,
-                                          float* __restrict__ C2x) {
+                                          float* __restrict__ C2x, int c_type) {
   const int64_t IN = I * N, q4 = IN / 4;
   const int64_t total = (int64_t)num_split[0] * q4;
   for (int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; x < total; x += (int64_t)gridDim.x * blockDim.x) {
@@ -316,10 +321,9 @@ __global__ void wgrad_chunk_reduce_kernel(const float* __restrict__ part, const 
     }
     for (; q < np; ++q) v += *reinterpret_cast<const f32x4*>(p0 + (int64_t)q * IN);
     const int64_t row = o / N, col = o % N;
-    float* dst;
-    if (e == x_expert) dst = (C2x && col >= n_split) ? C2x + row * ldc + (col - n_split) : Cx + row * ldc + col;
-    else dst = (C2 && col >= n_split) ? C2 + e * c_estride + row * ldc + (col - n_split) : C + e * c_estride + row * ldc + col;
-    *reinterpret_cast<f32x4*>(dst) = v;
+    const bool xe = e == x_expert, second = (xe ? C2x : C2) && col >= n_split;
+    store_grad4(xe ? (second ? C2x : Cx) : (second ? C2 : C), c_type,
+                (xe ? 0 : e * c_estride) + row * ldc + (second ? col - n_split : col), v);
   }
 }
 
@@ -540,15 +544,29 @@ size_t wgrad_workspace_bytes(int E, int64_t I, int64_t N, int S) {
   return S > 1 ? sizeof(float) * (size_t)S * E * I * N : 0;
 }
 
+// the 4-wave weight gradient on et operands, gradients in f32 or (c16) in et
+static int launch_wgrad_classic(int kid, unsigned grid, const WgradArgs& a, hipStream_t s, int et, bool c16) {
+  const dim3 g(grid), b(GT);
+  if (et == LSURGE_F16) {
+    if (c16) LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL((gemm_wgrad_kernel<Cfg, LSURGE_F16, true>), g, b, 0, s, a));
+    else LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL((gemm_wgrad_kernel<Cfg, LSURGE_F16>), g, b, 0, s, a));
+  } else {
+    if (c16) LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL((gemm_wgrad_kernel<Cfg, LSURGE_BF16, true>), g, b, 0, s, a));
+    else LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL(gemm_wgrad_kernel<Cfg>, g, b, 0, s, a));
+  }
+  return LSURGE_OK;
+}
+
 // C_e[I, N] = A_e^T @ B_e over the rows of expert e; columns >= n_split go to C2 (if given).  max_rows bounds
 // the rows of any one expert (the dense row count, or the token count for routed rows).
 int gemm_wgrad(int kid, int E, const int32_t* e_row0, int row0_mult, const int32_t* e_rows, int64_t dense_rows,
                int64_t max_rows, const void* A, int64_t lda, const void* B, int64_t ldb, int64_t I, int64_t N, float* C,
                float* C2, int64_t n_split, int64_t ldc, int64_t c_estride, int S, void* ws, size_t ws_bytes,
-               hipStream_t s, const RowGather& gather, int et) {
+               hipStream_t s, const RowGather& gather, int et, int c_type) {
   if (int rc = check_gemm_shape(I, N, "gemm_wgrad")) return rc;
   if (int rc = check_desc(max_rows * std::max(lda, ldb) * 2, "gemm_wgrad")) return rc;
   LSURGE_REQUIRE(S >= 1 && E >= 1, "gemm_wgrad: bad S/E");
+  LSURGE_REQUIRE(c_type == LSURGE_F32 || c_type == et, "gemm_wgrad: gradients must be f32 or of the operands' type");
   if (gather.rows) {
     LSURGE_REQUIRE(gather.div >= 1 && gather.nrows >= 1 && e_rows, "gemm_wgrad: bad row gather");
     if (int rc = check_desc(gather.nrows * lda * 2, "gemm_wgrad gather")) return rc;
@@ -567,11 +585,8 @@ int gemm_wgrad(int kid, int E, const int32_t* e_row0, int row0_mult, const int32
     a.part = (float*)ws;
   }
   const int64_t tiles = (int64_t)E * S * a.i_tiles * a.n_tiles;
-  if (et == LSURGE_F16)
-    LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL((gemm_wgrad_kernel<Cfg, LSURGE_F16>), dim3(pad8(tiles)), dim3(GT), 0, s, a));
-  else
-    LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL(gemm_wgrad_kernel<Cfg>, dim3(pad8(tiles)), dim3(GT), 0, s, a));
-  if (S > 1) return launch_splitk_reduce((const float*)ws, S, E, I, N, C, C2, n_split, ldc, c_estride, s);
+  if (int rc = launch_wgrad_classic(kid, pad8(tiles), a, s, et, c_type != LSURGE_F32)) return rc;
+  if (S > 1) return launch_splitk_reduce((const float*)ws, S, E, I, N, C, C2, n_split, ldc, c_estride, s, c_type);
   return LSURGE_OK;
 }
 
@@ -661,7 +676,7 @@ size_t wgrad_chunked_workspace_bytes(const WgradChunkPlan& p, int64_t I, int64_t
 int gemm_wgrad_chunked(int kid, const WgradChunks& ch, int E, int64_t max_rows, const void* A, int64_t lda,
                        const void* B, int64_t ldb, int64_t I, int64_t N, float* C, float* C2, int64_t n_split,
                        int64_t ldc, int64_t c_estride, void* part, size_t part_bytes, hipStream_t s,
-                       const RowGather& gather, const ExtraOut& xo, int et) {
+                       const RowGather& gather, const ExtraOut& xo, int et, int c_type) {
   if (int rc = check_gemm_shape(I, N, "gemm_wgrad_chunked")) return rc;
   LSURGE_REQUIRE(xo.expert < 0 || (xo.C && (xo.C2 || !C2)), "gemm_wgrad_chunked: extra expert outputs missing");
   if (int rc = check_desc(max_rows * std::max(lda, ldb) * 2, "gemm_wgrad_chunked")) return rc;
@@ -686,6 +701,8 @@ int gemm_wgrad_chunked(int kid, const WgradChunks& ch, int E, int64_t max_rows, 
   a.c_expert = ch.c_expert; a.c_row0 = ch.c_row0; a.c_rows = ch.c_rows; a.c_part = ch.c_part;
   a.num_chunks = ch.num_chunks; a.max_chunks = ch.max_chunks;
   a.x_expert = xo.expert; a.Cx = xo.C; a.C2x = xo.C2;
+  const bool c16 = c_type != LSURGE_F32;
+  LSURGE_REQUIRE(!c16 || c_type == et, "gemm_wgrad_chunked: gradients must be f32 or of the operands' type");
   // The persistent 256 x 256 kernel when a chunk has at least 16 tiles (the gate/up weight gradient: 16 per chunk at
   // d = 1024, 2f = 1024).  With fewer (the down weight gradient: 8 per chunk at f = 512, d = 1024) the persistent
   // grid gets about two tiles per workgroup and the last round leaves most CUs idle; the 4-wave 128 x 256 kernel,
@@ -698,31 +715,34 @@ int gemm_wgrad_chunked(int kid, const WgradChunks& ch, int E, int64_t max_rows, 
     a.i_tiles = (int)((I + g256::BM - 1) / g256::BM);
     a.n_tiles = (int)((N + g256::BN - 1) / g256::BN);
     const dim3 grid(g256::NWG), block(256);
+#define WG_LAUNCH(GATHER_, ET_, ONB_)                                                                                   \
+  do {                                                                                                                \
+    if (c16) LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL((g256::wgrad_kernel<GATHER_, ET_, ONB_, true>), grid, block, 0, s, a)); \
+    else LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL((g256::wgrad_kernel<GATHER_, ET_, ONB_>), grid, block, 0, s, a));    \
+  } while (0)
     if (et == LSURGE_F16) {
       LSURGE_REQUIRE(!a.a_rows, "gemm_wgrad_chunked: no row gather with f16 operands");
-      LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL((g256::wgrad_kernel<false, LSURGE_F16>), grid, block, 0, s, a));
+      WG_LAUNCH(false, LSURGE_F16, false);
     } else if (a.gather_b) {
-      LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL((g256::wgrad_kernel<true, LSURGE_BF16, true>), grid, block, 0, s, a));
+      WG_LAUNCH(true, LSURGE_BF16, true);
     } else if (a.a_rows) {
-      LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL((g256::wgrad_kernel<true>), grid, block, 0, s, a));
+      WG_LAUNCH(true, LSURGE_BF16, false);
     } else {
-      LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL((g256::wgrad_kernel<false>), grid, block, 0, s, a));
+      WG_LAUNCH(false, LSURGE_BF16, false);
     }
+#undef WG_LAUNCH
   } else {
     a.i_tiles = (int)((I + BM - 1) / BM);
     a.n_tiles = (int)((N + BN - 1) / BN);
     const int64_t tiles = (int64_t)pad8(ch.max_chunks) * a.i_tiles * a.n_tiles;  // see the chunk tile order
-    if (et == LSURGE_F16)
-      LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL((gemm_wgrad_kernel<Cfg, LSURGE_F16>), dim3((unsigned)tiles), dim3(GT), 0, s, a));
-    else
-      LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL(gemm_wgrad_kernel<Cfg>, dim3((unsigned)tiles), dim3(GT), 0, s, a));
+    if (int rc = launch_wgrad_classic(kid, (unsigned)tiles, a, s, et, c16)) return rc;
   }
   // grid-stride over the split experts' elements: two experts' worth of threads per pass
   const unsigned grid = (unsigned)std::min<int64_t>(2 * ((I * N / 4 + 255) / 256), 2048);
   LSURGE_LAUNCH(KID_SPLITK_REDUCE, s,
                 hipLaunchKernelGGL(wgrad_chunk_reduce_kernel, dim3(grid), dim3(256), 0, s, (const float*)part,
                                    ch.split_list, ch.num_split, ch.e_pbase, ch.e_nparts, I, N, C, C2, n_split, ldc,
-                                   c_estride, xo.expert, xo.C, xo.C2));
+                                   c_estride, xo.expert, xo.C, xo.C2, c_type));
   return LSURGE_OK;
 }
 
@@ -767,7 +787,7 @@ int gemm_wgrad_f8_chunked(int kid, const WgradChunks& ch, int E, int64_t max_row
   LSURGE_LAUNCH(KID_SPLITK_REDUCE, s,
                 hipLaunchKernelGGL(wgrad_chunk_reduce_kernel, dim3(grid), dim3(256), 0, s, (const float*)part,
                                    ch.split_list, ch.num_split, ch.e_pbase, ch.e_nparts, I, N, C, C2, n_split, ldc,
-                                   c_estride, -1, (float*)nullptr, (float*)nullptr));
+                                   c_estride, -1, (float*)nullptr, (float*)nullptr, (int)LSURGE_F32));
   return LSURGE_OK;
 }
 
@@ -1162,10 +1182,21 @@ int lsurge_ragged_dot_fp8(const void* lhs_q, const float* lhs_scale_inv, const v
 int lsurge_ragged_dot_bwd(const void* lhs, const void* rhs, const int32_t* group_sizes, const void* g, int64_t m,
                           int64_t kdim, int64_t n, int64_t e, int in_dtype, void* dlhs, float* drhs, void* workspace,
                           size_t workspace_bytes, lsurge_stream_t stream) {
+  return lsurge_ragged_dot_bwd_as(lhs, rhs, group_sizes, g, m, kdim, n, e, in_dtype, dlhs, drhs, LSURGE_F32, workspace,
+                                  workspace_bytes, stream);
+}
+
+int lsurge_ragged_dot_bwd_as(const void* lhs, const void* rhs, const int32_t* group_sizes, const void* g, int64_t m,
+                             int64_t kdim, int64_t n, int64_t e, int in_dtype, void* dlhs, void* drhs_out,
+                             int drhs_dtype, void* workspace, size_t workspace_bytes, lsurge_stream_t stream) {
+  float* drhs = (float*)drhs_out;  // 16-bit gradients: their own elements behind the same pointer
   LSURGE_REQUIRE(m >= 0 && e >= 1 && m < (1ll << 31), "ragged_dot_bwd: bad m/e");
   if (in_dtype != LSURGE_F32 && in_dtype != LSURGE_BF16 && in_dtype != LSURGE_F16)
     return lsurge::set_error(LSURGE_ERR_DTYPE, "ragged_dot_bwd: operands must be f32, bf16 or f16 (got dtype %d)",
                              in_dtype);
+  if (drhs_dtype != LSURGE_F32 && drhs_dtype != in_dtype)
+    return lsurge::set_error(LSURGE_ERR_DTYPE, "ragged_dot_bwd: drhs must be f32 or of the operands' dtype (got %d)",
+                             drhs_dtype);
   LSURGE_REQUIRE(lhs && rhs && group_sizes && g && dlhs && drhs, "ragged_dot_bwd: null pointer");
   hipStream_t s = (hipStream_t)stream;
   if (in_dtype == LSURGE_F32)
@@ -1197,10 +1228,10 @@ int lsurge_ragged_dot_bwd(const void* lhs, const void* rhs, const int32_t* group
     if (int rc = lsurge::build_wgrad_chunks(e_rows, e_row0, (int)e, p, table, &ch, s, -1, 0, 1)) return rc;
     return lsurge::gemm_wgrad_chunked(KID_MISC, ch, (int)e, m, lhs, kdim, g, n, kdim, n, drhs, nullptr, 0, n, kdim * n,
                                       base + off, lsurge::wgrad_chunked_workspace_bytes(p, kdim, n), s,
-                                      lsurge::RowGather(), lsurge::ExtraOut(), in_dtype);
+                                      lsurge::RowGather(), lsurge::ExtraOut(), in_dtype, drhs_dtype);
   }
   return lsurge::gemm_wgrad(KID_MISC, (int)e, e_row0, 1, e_rows, 0, m, lhs, kdim, g, n, kdim, n, drhs, nullptr, 0, n,
-                            kdim * n, 1, nullptr, 0, s, lsurge::RowGather(), in_dtype);
+                            kdim * n, 1, nullptr, 0, s, lsurge::RowGather(), in_dtype, drhs_dtype);
 }
 
 }  // extern "C"

@@ -552,7 +552,9 @@ void rows_kernel(RowsArgs a) {
 // ONB (with GATHER): the gather applies to B instead, and each gathered B row is multiplied by b_scale[r] (chunks of
 // x_expert: 1) and rounded to bf16 as it is staged into LDS (the layer's dY rows times their routing weight, the
 // operand the combine backward would otherwise write out); the weights ride along the row indices.
-template <bool GATHER, int ET = LSURGE_BF16, bool ONB = false>
+// C16: the gradients are written in ET, each f32 result rounded once (half the bytes of the epilogue, and no f32 copy
+// to convert afterwards).
+template <bool GATHER, int ET = LSURGE_BF16, bool ONB = false, bool C16 = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void wgrad_kernel(WgradArgs a) {
   __shared__ __attribute__((aligned(1024))) char smem[SMEM_BYTES];
@@ -731,8 +733,8 @@ void wgrad_kernel(WgradArgs a) {
   F f0, f1;
   fread(f0, 0, 0);
 
-  // ---- epilogue of tile t_cur (f32): the chunk's partial slot, or the gradient split at n_split -- two uniform
-  // destinations, lanes whose columns belong to the other one pass the out-of-range offset
+  // ---- epilogue of tile t_cur: the chunk's partial slot (f32), or the gradient (f32, or of type ET with C16) split at
+  // n_split -- two uniform destinations, lanes whose columns belong to the other one pass the out-of-range offset
   char* const stg = smem + RING_BYTES + wave * STG_BYTES;
   auto epilogue = [&]() {
     // the lane index, opaque to the compiler here (as in the row kernel's epilogue): the per-lane offsets below are
@@ -745,23 +747,26 @@ void wgrad_kernel(WgradArgs a) {
     const int expert = ctab(a.c_expert, c), part = ctab(a.c_part, c);
     const int64_t i0 = (int64_t)it * BM, n0 = (int64_t)nt * BN;
     const int64_t irows = min((int64_t)BM, (int64_t)I - i0);
-    const float* d1;
-    const float* d2 = nullptr;
+    const bool o16 = C16 && part < 0;
+    const int osh = o16 ? 1 : 2;  // log2 of the output's element size
+    const char* d1;
+    const char* d2 = nullptr;
     int64_t pitch, split;
     if (part >= 0) {
-      d1 = a.part + (int64_t)part * I * N;
+      d1 = reinterpret_cast<const char*>(a.part + (int64_t)part * I * N);
       pitch = N;
       split = N;
     } else {
       const bool xe = expert == a.x_expert;
-      d1 = xe ? a.Cx : a.C + (int64_t)expert * a.c_estride;
-      d2 = xe ? a.C2x : (a.C2 ? a.C2 + (int64_t)expert * a.c_estride : nullptr);
+      const int64_t eo = ((int64_t)expert * a.c_estride) << osh;
+      d1 = xe ? reinterpret_cast<const char*>(a.Cx) : reinterpret_cast<const char*>(a.C) + eo;
+      d2 = xe ? reinterpret_cast<const char*>(a.C2x) : (a.C2 ? reinterpret_cast<const char*>(a.C2) + eo : nullptr);
       pitch = a.ldc;
       split = d2 ? a.n_split : N;
     }
-    const rsrc_t r1 = rsrc(d1 + i0 * pitch, irows * pitch * 4);
-    const rsrc_t r2 = rsrc(d2 ? d2 + i0 * pitch : nullptr, d2 ? irows * pitch * 4 : 0);
-    const uint32_t pb = (uint32_t)pitch * 4u;
+    const rsrc_t r1 = rsrc(d1 + ((i0 * pitch) << osh), (irows * pitch) << osh);
+    const rsrc_t r2 = rsrc(d2 ? d2 + ((i0 * pitch) << osh) : nullptr, d2 ? (irows * pitch) << osh : 0);
+    const uint32_t pb = (uint32_t)pitch << osh;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int rbase = wm * 128 + 32 * i;
@@ -786,10 +791,17 @@ void wgrad_kernel(WgradArgs a) {
           const u32x4 v = *reinterpret_cast<const u32x4*>(stg + r * 256 + ((cc ^ (r & 15)) << 4));
           const int64_t col = seg + 4 * cc;
           const uint32_t rb = (uint32_t)(rbase + r) * pb;
-          const uint32_t o1 = col < split ? rb + (uint32_t)col * 4u : OOB;
-          const uint32_t o2 = col >= split && col < N ? rb + (uint32_t)(col - split) * 4u : OOB;
-          if (side != 1) __builtin_amdgcn_raw_buffer_store_b128(v, r1, o1, 0, 0);
-          if (side != 0) __builtin_amdgcn_raw_buffer_store_b128(v, r2, o2, 0, 0);
+          const uint32_t o1 = col < split ? rb + ((uint32_t)col << osh) : OOB;
+          const uint32_t o2 = col >= split && col < N ? rb + ((uint32_t)(col - split) << osh) : OOB;
+          if (o16) {
+            const uint2 h = pack_grad4(ET, __builtin_bit_cast(f32x4, v));
+            const u32x2 h2 = u32x2{h.x, h.y};
+            if (side != 1) __builtin_amdgcn_raw_buffer_store_b64(h2, r1, o1, 0, 0);
+            if (side != 0) __builtin_amdgcn_raw_buffer_store_b64(h2, r2, o2, 0, 0);
+          } else {
+            if (side != 1) __builtin_amdgcn_raw_buffer_store_b128(v, r1, o1, 0, 0);
+            if (side != 0) __builtin_amdgcn_raw_buffer_store_b128(v, r2, o2, 0, 0);
+          }
         }
       }
 #pragma unroll

@@ -153,6 +153,22 @@ struct WgradArgs {
   const float* a_sinv = nullptr;
   const float* b_sinv = nullptr;
 };
+// The gradients C, C2, Cx and C2x are f32, or 16-bit values of the operands' type behind the same pointers (the kernels'
+// C16 parameter, the reductions' c_type), rounded once from the f32 result.  Partials are always f32.
+
+// four f32 gradients -> element o of an output of type ct (o a multiple of 4)
+__device__ __forceinline__ uint2 pack_grad4(int ct, f32x4 v) {
+  if (ct == LSURGE_F16) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    return uint2{__builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){v[0], v[1]}, h2)),
+                 __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){v[2], v[3]}, h2))};
+  }
+  return uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+}
+__device__ __forceinline__ void store_grad4(float* C, int ct, int64_t o, f32x4 v) {
+  if (ct == LSURGE_F32) *reinterpret_cast<f32x4*>(C + o) = v;
+  else *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(C) + o) = pack_grad4(ct, v);
+}
 
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
@@ -789,7 +805,8 @@ void gemm_rows_kernel(RowsArgs a) {
 // Weight-gradient epilogue (f32), staged through LDS as in gemm_rows_kernel: acc[i][j][4q + t] is C row
 // i0 + wm*TM + 32 i + lane%32, column n0 + wn*TN + 32 j + 8 q + 4 (lane/32) + t.  Read back with TN/8 lanes per row,
 // each lane storing 8 contiguous f32, to the chunk's partial slot, the split partials, or the gradient itself.
-template <class Cfg>
+// C16: 16-bit gradients of type ET.
+template <class Cfg, bool C16 = false, int ET = LSURGE_BF16>
 __device__ __forceinline__ void wgrad_epilogue(const WgradArgs& a, const f32x16 (&acc)[Cfg::FM][Cfg::FN],
                                                bf16_t* smem, int wave, int lane, int64_t i0, int64_t n0,
                                                float* part_out, int S, int s, int e) {
@@ -813,14 +830,15 @@ __device__ __forceinline__ void wgrad_epilogue(const WgradArgs& a, const f32x16 
         const int64_t col = n0 + wn * TN + c + 4 * h;
         if (col >= N) continue;
         const f32x4 v = *reinterpret_cast<const f32x4*>(stg + r * SP + c + 4 * h);
-        float* dst;
-        if (part_out) dst = part_out + row * N + col;
-        else if (S > 1) dst = a.part + (((int64_t)s * a.E + e) * I + row) * N + col;
-        else if (e == a.x_expert) dst = (a.C2x && col >= a.n_split) ? a.C2x + row * a.ldc + (col - a.n_split)
-                                                                    : a.Cx + row * a.ldc + col;
-        else if (a.C2 && col >= a.n_split) dst = a.C2 + (int64_t)e * a.c_estride + row * a.ldc + (col - a.n_split);
-        else dst = a.C + (int64_t)e * a.c_estride + row * a.ldc + col;
-        *reinterpret_cast<f32x4*>(dst) = v;
+        if (part_out) {
+          *reinterpret_cast<f32x4*>(part_out + row * N + col) = v;
+        } else if (S > 1) {
+          *reinterpret_cast<f32x4*>(a.part + (((int64_t)s * a.E + e) * I + row) * N + col) = v;
+        } else {
+          const bool xe = e == a.x_expert, second = (xe ? a.C2x : a.C2) && col >= a.n_split;
+          store_grad4(xe ? (second ? a.C2x : a.Cx) : (second ? a.C2 : a.C), C16 ? ET : LSURGE_F32,
+                      (xe ? 0 : (int64_t)e * a.c_estride) + row * a.ldc + (second ? col - a.n_split : col), v);
+        }
       }
     }
   }
@@ -829,7 +847,7 @@ __device__ __forceinline__ void wgrad_epilogue(const WgradArgs& a, const f32x16 
 // =====================================================================================================
 // Weight gradient C_e[I, N] = A_e^T B_e, reduced over the rows of expert e: both operands are row-major
 // [rows, .] (the reduction dim is the slow one), so both are staged N-major and read with the transpose read.
-template <class Cfg, int ET = LSURGE_BF16>
+template <class Cfg, int ET = LSURGE_BF16, bool C16 = false>
 __global__ __launch_bounds__(Cfg::GT) __attribute__((amdgpu_waves_per_eu(Cfg::NW * Cfg::OCC / 4)))
 void gemm_wgrad_kernel(WgradArgs a) {
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, ST = Cfg::ST;
@@ -1005,7 +1023,7 @@ void gemm_wgrad_kernel(WgradArgs a) {
     else run_k_loop<Cfg, F>(nk, wave, issue, [](int, int, F&) {}, [](const F&) {});
   }
 
-  wgrad_epilogue<Cfg>(a, acc, smem, wave, lane, i0, n0, part_out, S, s, e);
+  wgrad_epilogue<Cfg, C16, ET>(a, acc, smem, wave, lane, i0, n0, part_out, S, s, e);
 }
 
 // =====================================================================================================

@@ -132,10 +132,12 @@ int gemm_rows_f8(int kid, const GemmBlocks& g, const void* A, int64_t lda, const
                  int64_t N, void* C, int64_t ldc, bool out_f32, int epi, void* Gs, void* Us, uint32_t* amax,
                  hipStream_t s, const RowGather& gather = RowGather(), int64_t k_split = 0, bool a_e5m2 = false);
 size_t wgrad_workspace_bytes(int E, int64_t I, int64_t N, int S);
+// weight gradients: c_type is the element type behind C, C2 (and an ExtraOut's): LSURGE_F32, or a 16-bit type rounded
+// once from the f32 result
 int gemm_wgrad(int kid, int E, const int32_t* e_row0, int row0_mult, const int32_t* e_rows, int64_t dense_rows,
                int64_t max_rows, const void* A, int64_t lda, const void* B, int64_t ldb, int64_t I, int64_t N,
                float* C, float* C2, int64_t n_split, int64_t ldc, int64_t c_estride, int S, void* ws, size_t ws_bytes,
-               hipStream_t s, const RowGather& gather = RowGather(), int et = LSURGE_BF16);
+               hipStream_t s, const RowGather& gather = RowGather(), int et = LSURGE_BF16, int c_type = LSURGE_F32);
 
 // Chunked routed weight gradient: every expert's rows cut into chunks of at most R rows (see WgradArgs), so a
 // hot expert spreads over many workgroups; split experts are reduced from f32 partial slots in chunk order.
@@ -174,7 +176,8 @@ size_t wgrad_chunked_workspace_bytes(const WgradChunkPlan& p, int64_t I, int64_t
 int gemm_wgrad_chunked(int kid, const WgradChunks& ch, int E, int64_t max_rows, const void* A, int64_t lda,
                        const void* B, int64_t ldb, int64_t I, int64_t N, float* C, float* C2, int64_t n_split,
                        int64_t ldc, int64_t c_estride, void* part, size_t part_bytes, hipStream_t s,
-                       const RowGather& gather = RowGather(), const ExtraOut& xo = ExtraOut(), int et = LSURGE_BF16);
+                       const RowGather& gather = RowGather(), const ExtraOut& xo = ExtraOut(), int et = LSURGE_BF16,
+                       int c_type = LSURGE_F32);
 
 // FP8 weight gradients (E4M3 activations x E5M2 gradients) from the row-major FP8 tensors: A [rows, lda] and B
 // [rows, ldb] bytes (A optionally gathered through row_src, as gemm_wgrad_chunked), C = A^T B a_sinv[0] b_sinv[0].

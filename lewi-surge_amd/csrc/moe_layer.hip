@@ -631,7 +631,15 @@ int lsurge_moe_fwd_fp8(const lsurge_moe_shape* s, const lsurge_moe_params* p, co
 // critical stream gets one record (the fork, shared by both helpers) and one wait (the join: s1 waits for s0 first).
 int lsurge_moe_bwd(const lsurge_moe_shape* s, const lsurge_moe_params* p, const void* dy, const void* saved,
                    const lsurge_moe_grads* g, void* workspace, size_t workspace_bytes, lsurge_stream_t stream) {
+  return lsurge_moe_bwd_as(s, p, dy, saved, g, LSURGE_F32, workspace, workspace_bytes, stream);
+}
+
+int lsurge_moe_bwd_as(const lsurge_moe_shape* s, const lsurge_moe_params* p, const void* dy, const void* saved,
+                      const lsurge_moe_grads* g, int dw_dtype, void* workspace, size_t workspace_bytes,
+                      lsurge_stream_t stream) {
   if (int rc = check_shape(s)) return rc;
+  if (dw_dtype != LSURGE_F32 && dw_dtype != LSURGE_BF16)
+    return lsurge::set_error(LSURGE_ERR_DTYPE, "moe_bwd: weight gradients must be f32 or bf16 (got dtype %d)", dw_dtype);
   LSURGE_REQUIRE(p && p->x && p->w_r && p->w_gate && p->w_up && p->w_down && dy && saved && g, "moe_bwd: null pointer");
   LSURGE_REQUIRE(g->dx && g->dw_r && g->dw_gate && g->dw_up && g->dw_down, "moe_bwd: null gradient pointer");
   LSURGE_REQUIRE(!s->fs || (p->ws_gate && p->ws_up && p->ws_down && g->dws_gate && g->dws_up && g->dws_down),
@@ -684,7 +692,7 @@ int lsurge_moe_bwd(const lsurge_moe_shape* s, const lsurge_moe_params* p, const 
       return rc;
     if (int rc = lsurge::gemm_wgrad_chunked(KID_SHARED_DOWN_WGRAD, dch, 0, q.T, sv.sh, q.fs, dy, q.d, q.fs, q.d,
                                             nullptr, nullptr, 0, q.d, 0, w.part, w.part_bytes, s0,
-                                            lsurge::RowGather(), dxo))
+                                            lsurge::RowGather(), dxo, LSURGE_BF16, dw_dtype))
       return rc;
     if (int rc = lsurge::gemm_rows_nk(KID_SHARED_GU_DGRAD, dense, w.sdgu, 2 * q.fs, p->ws_gate, p->ws_up, q.fs, q.fs, 0,
                                       2 * q.fs, q.d, w.sdx, q.d, false, nullptr, nullptr, 0, s0))
@@ -696,7 +704,7 @@ int lsurge_moe_bwd(const lsurge_moe_shape* s, const lsurge_moe_params* p, const 
       return rc;
     if (int rc = lsurge::gemm_wgrad_chunked(KID_SHARED_GU_WGRAD, dch, 0, q.T, p->x, q.d, w.sdgu, 2 * q.fs, q.d,
                                             2 * q.fs, nullptr, nullptr, q.fs, q.fs, 0, w.part, w.part_bytes, s0,
-                                            lsurge::RowGather(), dxo))
+                                            lsurge::RowGather(), dxo, LSURGE_BF16, dw_dtype))
       return rc;
   }
   // the chunk table of the routed weight gradients and W_r^T (the router's dx term) were made by the forward
@@ -739,7 +747,7 @@ int lsurge_moe_bwd(const lsurge_moe_shape* s, const lsurge_moe_params* p, const 
     if (int rc = lsurge::gemm_wgrad_chunked(KID_GEMM_DOWN_WGRAD, chunks, (int)q.E, q.T, sv.h, q.f,
                                             dy_rows ? (const void*)w.dy_pad : dy, q.d, q.f, q.d, g->dw_down, nullptr, 0,
                                             q.d, q.f * q.d, w.part_dn, w.part_dn_bytes, s1,
-                                            dy_rows ? lsurge::RowGather() : bg, odn))
+                                            dy_rows ? lsurge::RowGather() : bg, odn, LSURGE_BF16, dw_dtype))
       return rc;
   }
   // router backward dW_r = x^T dlogits (bf16 MFMA over the dense [T, E] dlogits): on s0 beside the down wgrad when
@@ -748,7 +756,8 @@ int lsurge_moe_bwd(const lsurge_moe_shape* s, const lsurge_moe_params* p, const 
   {
     const int S = dense_splits(q.T, q.d, q.E);
     if (int rc = lsurge::gemm_wgrad(KID_ROUTER_WGRAD, 1, nullptr, 1, nullptr, q.T, q.T, p->x, q.d, w.dlog, q.E, q.d,
-                                    q.E, g->dw_r, nullptr, 0, q.E, 0, S, w.part_r, w.part_r_bytes, sr))
+                                    q.E, g->dw_r, nullptr, 0, q.E, 0, S, w.part_r, w.part_r_bytes, sr,
+                                    lsurge::RowGather(), LSURGE_BF16, dw_dtype))
       return rc;
   }
   // main: down dgrad + SwiGLU backward: dH = dY_pad W_down^T, or w (dY W_down^T) from gathered dY rows -> [dG | dU]
@@ -774,7 +783,7 @@ int lsurge_moe_bwd(const lsurge_moe_shape* s, const lsurge_moe_params* p, const 
     gather.nrows = q.T;
     if (int rc = lsurge::gemm_wgrad_chunked(KID_GEMM_GU_WGRAD, chunks, (int)q.E, q.T, p->x, q.d, w.dgu, 2 * q.f, q.d,
                                             2 * q.f, g->dw_gate, g->dw_up, q.f, q.f, q.d * q.f, w.part_gu,
-                                            w.part_gu_bytes, st, gather, ogu))
+                                            w.part_gu_bytes, st, gather, ogu, LSURGE_BF16, dw_dtype))
       return rc;
   }
   // join all helpers (s1 after s0, the critical stream after s1) at the end: nothing on the critical stream reads

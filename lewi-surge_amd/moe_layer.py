@@ -132,16 +132,20 @@ class MoELayer:
                                        self._fwd8_ws.numel(), L.stream(self.device)), "moe_fwd_fp8")
         return out
 
-    def alloc_grads(self):
+    def alloc_grads(self, dw_dtype=torch.float32):
+        """Gradient buffers for backward(): dx bf16, dweights f32, the weight gradients in dw_dtype (f32 or bf16)."""
         s = self.shape
-        z = lambda *shape: torch.empty(shape, dtype=torch.float32, device=self.device)  # noqa: E731
+        z = lambda *shape: torch.empty(shape, dtype=dw_dtype, device=self.device)  # noqa: E731
         g = dict(dx=torch.empty((s.t, s.d), dtype=torch.bfloat16, device=self.device), dw_r=z(s.d, s.e),
-                 dw_gate=z(s.e, s.d, s.f), dw_up=z(s.e, s.d, s.f), dw_down=z(s.e, s.f, s.d), dweights=z(s.t, s.k))
+                 dw_gate=z(s.e, s.d, s.f), dw_up=z(s.e, s.d, s.f), dw_down=z(s.e, s.f, s.d),
+                 dweights=torch.empty((s.t, s.k), dtype=torch.float32, device=self.device))
         if s.fs:
             g.update(dws_gate=z(s.d, s.fs), dws_up=z(s.d, s.fs), dws_down=z(s.fs, s.d))
         return g
 
     def backward(self, p: dict, dy, grads=None):
+        """Gradients into `grads` (alloc_grads(); by default this layer's own f32 ones): weight gradients in their
+        buffers' dtype, float32 or bfloat16 (each f32 gradient rounded once)."""
         s = self.shape
         _check_params(s, p)
         if tuple(dy.shape) != (s.t, s.d) or dy.dtype != torch.bfloat16 or not dy.is_contiguous():
@@ -150,13 +154,16 @@ class MoELayer:
             if self.grads is None:
                 self.grads = self.alloc_grads()
             grads = self.grads
+        dw = [grads[n] for n in GRAD_NAMES if n.startswith("dw") and n != "dweights" and grads.get(n) is not None]
+        if len({t.dtype for t in dw}) > 1:
+            raise ValueError("moe_layer: the weight gradients must share one dtype")
         if self._bwd_ws is None:
             self._bwd_ws = L.workspace(L.lib().lsurge_moe_bwd_workspace_bytes(ctypes.byref(self._cs)), self.device)
         gs = L.MoeGrads(*[None if grads.get(n) is None else grads[n].data_ptr() for n in GRAD_NAMES])
         ps = _params_struct(p)
-        L.check(L.lib().lsurge_moe_bwd(ctypes.byref(self._cs), ctypes.byref(ps), L.ptr(dy), L.ptr(self.saved),
-                                       ctypes.byref(gs), L.ptr(self._bwd_ws), self._bwd_ws.numel(),
-                                       L.stream(self.device)), "moe_bwd")
+        L.check(L.lib().lsurge_moe_bwd_as(ctypes.byref(self._cs), ctypes.byref(ps), L.ptr(dy), L.ptr(self.saved),
+                                          ctypes.byref(gs), L.dt(dw[0]) if dw else L.F32, L.ptr(self._bwd_ws),
+                                          self._bwd_ws.numel(), L.stream(self.device)), "moe_bwd")
         return grads
 
     def backward_fp8(self, p: dict, dy, grads=None):
@@ -228,12 +235,10 @@ class _MoEFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy):
-        g = ctx.layer.backward(ctx.p, L.contig(dy.to(torch.bfloat16)))
-        p = ctx.p
-        cast = lambda name, ref: None if ref is None else g[name].to(ref.dtype)  # noqa: E731
-        return (None, None, g["dx"], cast("dw_r", p["w_r"]), cast("dw_gate", p["w_gate"]), cast("dw_up", p["w_up"]),
-                cast("dw_down", p["w_down"]), cast("dws_gate", p["ws_gate"]), cast("dws_up", p["ws_up"]),
-                cast("dws_down", p["ws_down"]))
+        # the weights are bf16, so their gradients are written in bf16, into buffers of this call's own
+        g = ctx.layer.backward(ctx.p, L.contig(dy.to(torch.bfloat16)), ctx.layer.alloc_grads(torch.bfloat16))
+        return (None, None, g["dx"], g["dw_r"], g["dw_gate"], g["dw_up"], g["dw_down"], g.get("dws_gate"),
+                g.get("dws_up"), g.get("dws_down"))
 
 
 def moe_layer(x, w_r, w_gate, w_up, w_down, ws_gate=None, ws_up=None, ws_down=None, bias=None, k=6):

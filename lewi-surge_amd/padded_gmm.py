@@ -105,17 +105,17 @@ class _RaggedDot(torch.autograd.Function):
         e, _, n = rhs.shape
         g = L.contig(g.to(lhs.dtype))
         dlhs = torch.empty_like(lhs)
-        drhs = torch.empty((e, k, n), dtype=torch.float32, device=lhs.device)
+        drhs = torch.empty((e, k, n), dtype=rhs.dtype, device=lhs.device)  # rounded once from the f32 sums
         if lhs.dtype == torch.float32:
             g = _aligned(g)
             wsb = L.lib().lsurge_ragged_dot_bwd_f32_workspace_bytes(m, k, n, e)
         else:
             wsb = L.lib().lsurge_ragged_dot_bwd_workspace_bytes(m, k, n, e)
         ws = L.workspace(wsb, lhs.device)
-        L.check(L.lib().lsurge_ragged_dot_bwd(L.ptr(lhs), L.ptr(rhs), L.ptr(gs), L.ptr(g), m, k, n, e, L.dt(lhs),
-                                              L.ptr(dlhs), L.ptr(drhs), L.ptr(ws), ws.numel(), L.stream(lhs.device)),
-                "ragged_dot_bwd")
-        return dlhs, drhs.to(rhs.dtype), None, None
+        L.check(L.lib().lsurge_ragged_dot_bwd_as(L.ptr(lhs), L.ptr(rhs), L.ptr(gs), L.ptr(g), m, k, n, e, L.dt(lhs),
+                                                 L.ptr(dlhs), L.ptr(drhs), L.dt(drhs), L.ptr(ws), ws.numel(),
+                                                 L.stream(lhs.device)), "ragged_dot_bwd")
+        return dlhs, drhs, None, None
 
 
 def padded_ragged_dot(lhs, rhs, group_sizes, precision=None, preferred_element_type=None, **kw):

@@ -104,3 +104,60 @@ def test_layer_bitwise(T, d, E, k, f, fs, zipf, dev):
     for name in res[0]:
         x0, x1 = res[0][name], res[1][name]
         assert torch.equal(x0, x1), f"{name}: max |diff| {(x0.float() - x1.float()).abs().max().item()}"
+
+
+@pytest.mark.parametrize("M,K,N,E,hot,dtype", [(1000, 64, 72, 8, 0, torch.bfloat16), (3000, 512, 520, 4, 2600, torch.bfloat16),
+                                               (2304, 1024, 1024, 8, 0, torch.bfloat16), (700, 136, 256, 300, 0, torch.bfloat16),
+                                               (9000, 256, 264, 2, 8900, torch.float16), (640, 128, 128, 8, 0, torch.float16)])
+def test_ragged_dot_bwd_16bit_drhs(M, K, N, E, hot, dtype, dev):
+    """drhs in the operands' dtype is the f32 drhs rounded once, bit for bit: both kernel families, single chunks, split
+    hot groups (partials summed in f32 first), the unchunked path (300 groups), column remainders, empty groups."""
+    gen = torch.Generator(device=dev).manual_seed(M + N)
+    lhs = torch.randn((M, K), device=dev, generator=gen).to(dtype)
+    rhs = torch.randn((E, K, N), device=dev, generator=gen).to(dtype)
+    g = torch.randn((M, N), device=dev, generator=gen).to(dtype)
+    gs = torch.zeros(E, dtype=torch.int32)
+    gs[0] = hot
+    rest = M - hot - 5  # five rows past the groups
+    gs[1:-1 if E > 2 else E] += rest // (E - 2 if E > 2 else 1)
+    gs = gs.to(dev)
+    lib = _lib.lib()
+    ws = _lib.workspace(lib.lsurge_ragged_dot_bwd_workspace_bytes(M, K, N, E), dev)
+    for variant in (0, 1):
+        lib.lsurge_set_gemm_variant(variant)
+        try:
+            out = {}
+            for dt in (torch.float32, dtype):
+                dl = torch.empty((M, K), dtype=dtype, device=dev)
+                dr = torch.full((E, K, N), float("nan"), dtype=dt, device=dev)
+                _lib.check(lib.lsurge_ragged_dot_bwd_as(_lib.ptr(lhs), _lib.ptr(rhs), _lib.ptr(gs), _lib.ptr(g), M, K, N, E, _lib.dt(lhs),
+                                                     _lib.ptr(dl), _lib.ptr(dr), _lib.dt(dr), _lib.ptr(ws), ws.numel(),
+                                                     _lib.stream(dev)), "ragged_dot_bwd_as")
+                out[dt] = dr
+            assert torch.equal(out[torch.float32].to(dtype).view(torch.int16), out[dtype].view(torch.int16))
+        finally:
+            lib.lsurge_set_gemm_variant(1)
+    rc = lib.lsurge_ragged_dot_bwd_as(_lib.ptr(lhs), _lib.ptr(rhs), _lib.ptr(gs), _lib.ptr(g), M, K, N, E, _lib.dt(lhs), _lib.ptr(dl),
+                                      _lib.ptr(dr), _lib.F16 if dtype == torch.bfloat16 else _lib.BF16, _lib.ptr(ws), ws.numel(),
+                                      _lib.stream(dev))
+    assert rc == -2  # a 16-bit dtype other than the operands'
+
+
+@pytest.mark.parametrize("T,d,E,k,f,fs", [(1000, 256, 16, 4, 128, 128), (700, 512, 32, 6, 256, 1024), (900, 1024, 8, 2, 1024, 0)])
+def test_layer_backward_bf16_weight_gradients(T, d, E, k, f, fs, dev):
+    """Layer weight gradients written in bf16 are the f32 ones rounded once; dx and dweights do not change."""
+    p = mo.make_inputs(T=T, d=d, E=E, k=k, f=f, fs=fs, seed=3)
+    tp = {n: torch.from_numpy(p[n]).to(dev).to(torch.bfloat16) for n in
+          ("x", "w_r", "w_gate", "w_up", "w_down") + (("ws_gate", "ws_up", "ws_down") if fs else ())}
+    dy = torch.from_numpy(p["dy"]).to(dev).to(torch.bfloat16)
+    layer = MoELayer(MoEShape(T, d, E, k, f, fs), dev)
+    layer.forward(tp)
+    g32 = layer.backward(tp, dy)
+    g16 = layer.backward(tp, dy, layer.alloc_grads(torch.bfloat16))
+    for n, t in g32.items():
+        same = g16[n] if n in ("dx", "dweights") else g16[n].view(torch.int16)
+        want = t if n in ("dx", "dweights") else t.to(torch.bfloat16).view(torch.int16)
+        assert torch.equal(same, want), n
+    mixed = dict(layer.alloc_grads(), dw_down=g16["dw_down"])
+    with pytest.raises(ValueError, match="one dtype"):
+        layer.backward(tp, dy, mixed)
