@@ -74,14 +74,19 @@ __device__ __forceinline__ uint32_t bf16_hi_lo(float x, uint32_t* lo) {
   *lo = f32_to_bf16(x - bf16_to_f32(h));
   return h;
 }
+// two f32 -> packed hi pair (returned) and lo pair
+__device__ __forceinline__ uint32_t hi_lo2(float a, float b, uint32_t* lo) {
+  const uint32_t h = pack_bf16x2(a, b);
+  *lo = pack_bf16x2(a - __uint_as_float(h << 16), b - __uint_as_float(h & 0xffff0000u));
+  return h;
+}
 // four f32 -> hi and lo bf16 quads, 8-byte stores at two row-major places
 __device__ __forceinline__ void store_hi_lo4(bf16_t* hi, bf16_t* lo, const float* x) {
-  uint32_t l[4], h[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) h[i] = bf16_hi_lo(x[i], &l[i]);
   typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-  *reinterpret_cast<u32x2*>(hi) = u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
-  *reinterpret_cast<u32x2*>(lo) = u32x2{l[0] | (l[1] << 16), l[2] | (l[3] << 16)};
+  uint32_t l0, l1;
+  const uint32_t h0 = hi_lo2(x[0], x[1], &l0), h1 = hi_lo2(x[2], x[3], &l1);
+  *reinterpret_cast<u32x2*>(hi) = u32x2{h0, h1};
+  *reinterpret_cast<u32x2*>(lo) = u32x2{l0, l1};
 }
 
 // eight f32 -> bf16 fragment, and its hi / lo split
@@ -384,19 +389,32 @@ __global__ __launch_bounds__(GTH) void gdn_chunk_kernel(const bf16_t* __restrict
   }
 }
 
-// Scan over the chunks of one (32 value columns, head, sequence), on the matrix cores.  Eight waves:
-//   waves 4-7 hold the state slice S [128 x 32] in their accumulators (rows 32 (wave - 4) .., one 32 x 32 tile each),
-//   waves 0-1 form w S (rows 32 wave ..) and v_new = u - w S, waves 2-3 form (q e^gcum) S and o = that + attn v_new.
-// Per chunk, three phases between barriers:
-//   A  every thread stages its prefetched share of q (scaled), k, w, attn (hi / lo) and u in LDS;
-//   B  waves 0-3: w S or q S (K = 128); v_new to LDS as hi / lo, and e^(gcum_last - gcum) v_new for the update;
-//   C  waves 2-3: o = (q S) e^gcum + attn v_new; waves 4-7: S = e^gcum_last S + k^T (e^(gcum_last - gcum) v_new),
-//      then the new state to LDS (hi / lo, transposed) for the next chunk's phase B.
-// The next chunk's tiles load into registers while a wave is otherwise idle: waves 4-7 during phase B, waves 2-3
-// after their phase-B products, waves 0-1 during phase C.  LDS fragments of the next 16-deep step are read before
-// the MFMAs of the current one, and the hi and lo products of a phase accumulate in two independent chains.
+// LDS is what a scan's waves exchange: wait for this wave's LDS accesses, then for the workgroup.  The loads in flight
+// (two chunks ahead) stay in flight, which a release fence's full wait would not allow.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Scan over the chunks of one (32 value columns, head, sequence), on the matrix cores.  Eight waves, three roles:
+//   waves 0-1 (token rows 32 wave ..)       v_new = u - w S, to LDS as hi / lo and scaled by e^(gcum_last - gcum);
+//   waves 2-3 (token rows 32 (wave - 2) ..) o = (q e^gcum) S + attn v_new;
+//   waves 4-7 (state rows 32 (wave - 4) ..) hold the state slice S [128 x 32] in their accumulators, one 32 x 32 tile
+//                                           each: S = e^gcum_last S + k^T (e^(gcum_last - gcum) v_new), then S to LDS
+//                                           (hi / lo, transposed) for the next chunk.
+// Per chunk two phases: w S and q S and v_new | attn v_new and the state update, with a barrier before each.  The chain
+// from chunk to chunk is w S -> v_new -> update -> state in LDS; everything else is kept off it:
+//   - w and u are operands of one wave only, which loads its own MFMA fragments of w from memory into registers (a
+//     lane's 16 bytes of a row); k goes through a piece of LDS that only its wave touches (for the transpose read);
+//   - waves 4-7, idle in the first phase, use it to stage the next chunk's scaled q, this chunk's attn (hi / lo) and
+//     their k, and to store the state for the backward;
+//   - e^gcum of the token rows passes from waves 0-1 to waves 2-3 through LDS;
+//   - loads run two chunks ahead in two register sets, and the barriers wait for LDS accesses only.
+// What is left in the chain of a chunk is 16 + 8 MFMAs, their operand reads (all of a phase's issued at once) and the
+// hi / lo conversions in between; by counters the phases are bound by vector instruction issue (about 2000 wave
+// instructions a chunk) and LDS accesses (1900 cycles a chunk), so addresses are scalar bases with one lane offset.
+// Before: every tile staged through LDS by all threads in a third phase of each chunk.  Before -> after: 88 -> 62 us
+// for one sequence of 2048 tokens (32 workgroups), 283 -> 240 us at 8 x 4096 tokens with the states stored (where the
+// stores cost 80 us).  A version whose waves 2-3 loaded, scaled and split their own q and attn was bound by those two
+// waves (72 us).
 constexpr int KP = GC + 8;  // pitch of the [.][GC] bf16 tiles (144 bytes)
-constexpr int UP = SB + 8;  // pitch of the u tile [GC][SB] (80 bytes)
 __global__ __launch_bounds__(GTH) void gdn_scan_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                                                        const bf16_t* __restrict__ u_in, const bf16_t* __restrict__ w_in,
                                                        const float* __restrict__ attn_in,
@@ -404,209 +422,284 @@ __global__ __launch_bounds__(GTH) void gdn_scan_kernel(const bf16_t* __restrict_
                                                        float qscale, const float* __restrict__ h0,
                                                        bf16_t* __restrict__ o, float* __restrict__ h_out,
                                                        float* __restrict__ h_chunks = nullptr) {
-  __shared__ __attribute__((aligned(16))) bf16_t qs[GC][GP], ws[GC][GP], ks[GC][GP];  // [t][d]
-  __shared__ __attribute__((aligned(16))) bf16_t ah[GC][KP], al[GC][KP];             // attn hi / lo [t][j]
-  __shared__ __attribute__((aligned(16))) bf16_t shh[SB][GP], shl[SB][GP];           // state hi / lo [c][d]
-  __shared__ __attribute__((aligned(16))) bf16_t vh[SB][KP], vl[SB][KP];             // v_new hi / lo [c][t]
-  __shared__ __attribute__((aligned(16))) bf16_t vkh[SB][KP], vkl[SB][KP];           // e^(gl - g) v_new [c][t]
-  __shared__ __attribute__((aligned(16))) bf16_t us[GC][UP];                          // u [t][c]
-  __shared__ float gc[GC], ek[GC];  // gcum, exp(gcum_last - gcum)
+  __shared__ __attribute__((aligned(16))) bf16_t shh[SB][GP], shl[SB][GP];  // state hi / lo [c][d]
+  __shared__ __attribute__((aligned(16))) bf16_t vh[SB][KP], vl[SB][KP];    // v_new hi / lo [c][t]
+  __shared__ __attribute__((aligned(16))) bf16_t vkh[SB][KP], vkl[SB][KP];  // e^(gl - g) v_new [c][t]
+  __shared__ __attribute__((aligned(16))) bf16_t ks[GC][GP];                // k [t][d], a wave's 32 columns each
+  __shared__ __attribute__((aligned(16))) bf16_t qs[2][GC][GP];             // scaled q of a chunk (n % 2)
+  __shared__ __attribute__((aligned(16))) bf16_t ah[GC][KP], al[GC][KP];    // attn hi / lo [t][j]
+  __shared__ __attribute__((aligned(16))) float egs[2][GC];                 // e^gcum of a chunk's rows (n % 2)
   int cb, h, b;
   scan_ids(cb, h, b);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lc = lane & 31, lh = lane >> 5;  // this lane's column of a 32 x 32 tile, and its row quad offset (x 4)
   const int64_t row0 = (int64_t)b * T;
   const int64_t bh = (int64_t)b * H + h;
   // tile rows of this lane's accumulators: row(r) = rb + 8 (r / 4) + 4 lh + r % 4 (tokens for waves 0-3, state rows
   // for waves 4-7)
   const int rb = wave < 4 ? 32 * (wave & 1) : 32 * (wave - 4);
-  f32x16 acc = {};  // waves 4-7: the state tile; waves 0-3: this chunk's product
-  // waves 4-7: the state entering the next chunk to LDS (hi / lo, transposed)
-  auto put_state = [&]() {
-#pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4) {
-      const int d = rb + 8 * q4 + 4 * lh;
-      const float sv[4] = {acc[4 * q4], acc[4 * q4 + 1], acc[4 * q4 + 2], acc[4 * q4 + 3]};
-      store_hi_lo4(&shh[lc][d], &shl[lc][d], sv);
-    }
+  auto trow = [&](int n, int i) { return (row0 + min(n * GC + i, T - 1)) * H + h; };  // q / k / o row of token i
+  // gcum of this lane's 16 accumulator rows, and of the chunk's last row
+  struct Gates {
+    f32x4 g[4];
+    float last;
   };
-  if (wave >= 4) {
+  auto load_gates = [&](Gates& x, int n) {
+    const float* src = gcum_in + (bh * N + n) * GC;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int d = rb + 8 * (r / 4) + 4 * lh + r % 4;
-      acc[r] = h0 ? h0[(bh * GD + d) * GD + cb + lc] : 0.f;
-    }
-    put_state();
-  }
-  // This thread's share of the next chunk's tiles: two 16-byte pieces of each of q, k and w (piece e = tid + GTH p:
-  // row e / 16, columns 8 (e % 16)), eight attn values, (threads < GC) one gcum value and (waves 4-7) 8 u values
-  // (row (tid - 256) / 4, columns 8 ((tid - 256) % 4)).
-  constexpr int PP = GC * (GD / 8) / GTH;  // pieces per thread and tile
-  static_assert(PP * GTH == GC * (GD / 8) && GC * GC == 8 * GTH && GC * SB / 8 == GTH / 2, "scan tile split");
-  u32x4 pq[PP], pk[PP], pw[PP], pu = {0u, 0u, 0u, 0u};
-  f32x4 pa[2];
-  float pg = 0.f;
-  auto fetch = [&](int n) {
-    const int t0 = n * GC;
-    const int64_t chunk_id = bh * N + n;
-#pragma unroll
-    for (int p = 0; p < PP; ++p) {
-      const int e = tid + GTH * p, i = e / (GD / 8), c = 8 * (e % (GD / 8));
-      const bool in = t0 + i < T;
-      const int64_t off = ((row0 + t0 + i) * H + h) * GD + c;
-      pq[p] = in ? *reinterpret_cast<const u32x4*>(q + off) : u32x4{0u, 0u, 0u, 0u};
-      pk[p] = in ? *reinterpret_cast<const u32x4*>(k + off) : u32x4{0u, 0u, 0u, 0u};
-      pw[p] = *reinterpret_cast<const u32x4*>(w_in + chunk_id * GC * GD + i * GD + c);
-    }
-    const float* asrc = attn_in + chunk_id * GC * GC;
-    pa[0] = *reinterpret_cast<const f32x4*>(asrc + 4 * tid);
-    pa[1] = *reinterpret_cast<const f32x4*>(asrc + 4 * (tid + GTH));
-    if (tid < GC) pg = gcum_in[chunk_id * GC + tid];
-    if (wave >= 4) {
-      const int e = tid - GTH / 2;
-      pu = *reinterpret_cast<const u32x4*>(u_in + chunk_id * GC * GD + (e / (SB / 8)) * GD + cb + 8 * (e % (SB / 8)));
-    }
+    for (int q4 = 0; q4 < 4; ++q4) x.g[q4] = *reinterpret_cast<const f32x4*>(src + rb + 8 * q4 + 4 * lh);
+    x.last = src[GC - 1];
   };
-  fetch(0);
-  for (int n = 0; n < N; ++n) {
-    const int t0 = n * GC;
-    __syncthreads();  // the previous chunk is done with every LDS tile
+  // P S of one chunk: P's fragments of the eight 16-deep steps in registers, S hi / lo from LDS (all reads issued before
+  // the first MFMA needs one), hi and lo products in two independent chains
+  auto times_state = [&](const bf16x8 (&pf)[GD / 16]) {
+    bf16x8 fh[GD / 16], fl[GD / 16];
 #pragma unroll
-    for (int p = 0; p < PP; ++p) {
-      const int e = tid + GTH * p, i = e / (GD / 8), c = 8 * (e % (GD / 8));
-      float f[8];
-      unpack8g(pq[p], f);  // q * scale in the compute dtype (gdn_fast.py:56-57)
-      *reinterpret_cast<u32x4*>(&qs[i][c]) =
-          u32x4{pack_bf16x2(f[0] * qscale, f[1] * qscale), pack_bf16x2(f[2] * qscale, f[3] * qscale),
-                pack_bf16x2(f[4] * qscale, f[5] * qscale), pack_bf16x2(f[6] * qscale, f[7] * qscale)};
-      *reinterpret_cast<u32x4*>(&ks[i][c]) = pk[p];
-      *reinterpret_cast<u32x4*>(&ws[i][c]) = pw[p];
+    for (int j = 0; j < GD / 16; ++j) {
+      fh[j] = frag_row<GP>(&shh[0][0], lc, 16 * j + 8 * lh);
+      fl[j] = frag_row<GP>(&shl[0][0], lc, 16 * j + 8 * lh);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    f32x16 acc = {}, acc2 = {};
+#pragma unroll
+    for (int j = 0; j < GD / 16; ++j) {
+      acc = mma_bf16(pf[j], fh[j], acc);
+      acc2 = mma_bf16(pf[j], fl[j], acc2);
     }
 #pragma unroll
-    for (int hlf = 0; hlf < 2; ++hlf) {
-      const int e = 4 * (tid + GTH * hlf);
-      const float av[4] = {pa[hlf][0], pa[hlf][1], pa[hlf][2], pa[hlf][3]};
-      store_hi_lo4(&ah[e / GC][e % GC], &al[e / GC][e % GC], av);
+    for (int r = 0; r < 16; ++r) acc[r] += acc2[r];
+    return acc;
+  };
+  // chunk(set, n) for every chunk, the two register sets in turn
+  auto all_chunks = [&](auto& sets, auto&& chunk) {
+    int n = 0;
+    for (; n + 1 < N; n += 2) {
+      chunk(sets[0], n);
+      chunk(sets[1], n + 1);
     }
-    if (tid < GC) {  // wave 0: gcum and exp(gcum_last - gcum)
-      gc[tid] = pg;
-      ek[tid] = __expf(__shfl(pg, GC - 1, 64) - pg);
+    if (n < N) chunk(sets[0], n);
+  };
+
+  if (wave < 2) {
+    struct Set {
+      bf16x8 w[GD / 16];
+      bf16_t u[16];
+      Gates g;
+      float gr;  // gcum of row rb + lc
+    } sets[2];
+    auto load_w = [&](Set& x, int n) {
+      const bf16_t* src = w_in + ((bh * N + n) * GC + rb + lc) * GD + 8 * lh;
+#pragma unroll
+      for (int j = 0; j < GD / 16; ++j) x.w[j] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(src + 16 * j));
+    };
+    auto load_u = [&](Set& x, int n) {
+      const bf16_t* src = u_in + (bh * N + n) * GC * GD;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) x.u[r] = (src + (8 * (r / 4) + r % 4) * GD)[(uint32_t)(rb + 4 * lh) * GD + cb + lc];
+      load_gates(x.g, n);
+      x.gr = gcum_in[(bh * N + n) * GC + rb + lc];
+    };
+    auto chunk = [&](Set& x, int n) {
+      const int n2 = min(n + 2, N - 1);
+      egs[n & 1][rb + lc] = __expf(x.gr);
+      float ek[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) ek[r] = __expf(x.g.last - x.g.g[r / 4][r % 4]);
+      lds_barrier();  // the state entering chunk n is in LDS
+      const f32x16 acc = times_state(x.w);
+      load_w(x, n2);
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        const int t = rb + 8 * q4 + 4 * lh;
+        float vv[4], vk[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          vv[e] = bf16_to_f32(x.u[4 * q4 + e]) - acc[4 * q4 + e];
+          vk[e] = vv[e] * ek[4 * q4 + e];
+        }
+        store_hi_lo4(&vh[lc][t], &vl[lc][t], vv);
+        store_hi_lo4(&vkh[lc][t], &vkl[lc][t], vk);
+      }
+      lds_barrier();  // v_new is in LDS
+      load_u(x, n2);
+    };
+    load_w(sets[0], 0);
+    load_u(sets[0], 0);
+    load_w(sets[1], min(1, N - 1));
+    load_u(sets[1], min(1, N - 1));
+    all_chunks(sets, chunk);
+  } else if (wave < 4) {
+    const uint32_t opitch = (uint32_t)H * GD;                           // elements between tokens of o
+    const uint32_t olane = (uint32_t)(rb + 4 * lh) * opitch + cb + lc;  // this lane's element of a chunk's row block
+    for (int n = 0; n < N; ++n) {
+      lds_barrier();  // the state entering chunk n is in LDS
+      bf16x8 pf[GD / 16];
+#pragma unroll
+      for (int j = 0; j < GD / 16; ++j) pf[j] = frag_row<GP>(&qs[n & 1][0][0], rb + lc, 16 * j + 8 * lh);
+      f32x16 acc = times_state(pf);
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        const f32x4 eg = *reinterpret_cast<const f32x4*>(&egs[n & 1][rb + 8 * q4 + 4 * lh]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[4 * q4 + e] *= eg[e];
+      }
+      lds_barrier();  // v_new is in LDS
+      // + attn v_new (attn is zero above the diagonal), K = 64
+      bf16x8 ph[GC / 16], pl[GC / 16], qh[GC / 16], ql[GC / 16];
+#pragma unroll
+      for (int j = 0; j < GC / 16; ++j) {
+        ph[j] = frag_row<KP>(&ah[0][0], rb + lc, 16 * j + 8 * lh);
+        qh[j] = frag_row<KP>(&vh[0][0], lc, 16 * j + 8 * lh);
+        ql[j] = frag_row<KP>(&vl[0][0], lc, 16 * j + 8 * lh);
+        pl[j] = frag_row<KP>(&al[0][0], rb + lc, 16 * j + 8 * lh);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      f32x16 acc2 = {};
+#pragma unroll
+      for (int j = 0; j < GC / 16; ++j) {
+        acc = mma_bf16(ph[j], qh[j], acc);
+        acc2 = mma_bf16(ph[j], ql[j], acc2);
+        acc2 = mma_bf16(pl[j], qh[j], acc2);
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[r] += acc2[r];
+      if (o) {  // the backward's recompute needs the states only
+        // scalar row bases, one 32-bit lane offset; only a sequence's last chunk can miss rows
+        bf16_t* ob = o + ((row0 + (int64_t)n * GC) * H + h) * GD;
+        const int left = T - n * GC - rb;  // rows from the tile's first (uniform)
+        if (left >= 32) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) (ob + (8 * (r / 4) + r % 4) * (int64_t)opitch)[olane] = f32_to_bf16(acc[r]);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            if (8 * (r / 4) + 4 * lh + r % 4 < left)
+              (ob + (8 * (r / 4) + r % 4) * (int64_t)opitch)[olane] = f32_to_bf16(acc[r]);
+        }
+      }
     }
-    if (wave >= 4) {
-      const int e = tid - GTH / 2;
-      *reinterpret_cast<u32x4*>(&us[e / (SB / 8)][8 * (e % (SB / 8))]) = pu;
-      if (h_chunks)  // the state entering chunk n, for the backward (issued here, after this phase's load wait)
+  } else {
+    struct Set {  // of chunk n: its k, its attn and the next chunk's q
+      u32x4 k[4], q[4];
+      f32x4 a[4];
+      float last;
+    } sets[2];
+    // this thread's share of q and attn: pieces e = ts + 256 p, row e / 16, columns 8 (e % 16) / 4 (e % 16)
+    const int ts = tid - GTH / 2, er = ts >> 4, ec = ts & 15;
+    const int qpitch = H * GD;  // elements between tokens of q and k
+    auto load_q = [&](Set& x, int n) {
+      if (n * GC + GC <= T) {  // scalar row bases, one 32-bit lane offset
+        const bf16_t* src = q + ((row0 + (int64_t)n * GC) * H + h) * GD;
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+          x.q[p] = *reinterpret_cast<const u32x4*>(src + 16 * p * (int64_t)qpitch + (uint32_t)(er * qpitch + 8 * ec));
+      } else {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) x.q[p] = *reinterpret_cast<const u32x4*>(q + trow(n, er + 16 * p) * GD + 8 * ec);
+      }
+    };
+    auto put_q = [&](const Set& x, int n) {  // q * scale in the compute dtype (gdn_fast.py:56-57)
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        float f[8];
+        unpack8g(x.q[p], f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] *= qscale;
+        *reinterpret_cast<bf16x8*>(&qs[n & 1][er + 16 * p][8 * ec]) = pack8(f);
+      }
+    };
+    auto load_a = [&](Set& x, int n) {
+      const float* src = attn_in + (bh * N + n) * GC * GC + 4 * ts;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) x.a[p] = *reinterpret_cast<const f32x4*>(src + 1024 * p);
+    };
+    // k columns rb .. + 31: piece p is row 16 p + lane / 4, columns rb + 8 (lane % 4)
+    const int kr = lane >> 2, kc = rb + 8 * (lane & 3);
+    auto load_k = [&](Set& x, int n) {
+      if (n * GC + GC <= T) {
+        const bf16_t* src = k + ((row0 + (int64_t)n * GC) * H + h) * GD;
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+          x.k[p] = *reinterpret_cast<const u32x4*>(src + 16 * p * (int64_t)qpitch + (uint32_t)(kr * qpitch + kc));
+      } else {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) x.k[p] = *reinterpret_cast<const u32x4*>(k + trow(n, 16 * p + kr) * GD + kc);
+      }
+      x.last = gcum_in[(bh * N + n) * GC + GC - 1];
+    };
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      acc[r] = h0 ? h0[(bh * GD + rb + 8 * (r / 4) + 4 * lh + r % 4) * GD + cb + lc] : 0.f;
+    // the state entering the next chunk to LDS (hi / lo, transposed)
+    auto put_state = [&]() {
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        const int d = rb + 8 * q4 + 4 * lh;
+        const float sv[4] = {acc[4 * q4], acc[4 * q4 + 1], acc[4 * q4 + 2], acc[4 * q4 + 3]};
+        store_hi_lo4(&shh[lc][d], &shl[lc][d], sv);
+      }
+    };
+    auto chunk = [&](Set& x, int n) {
+      lds_barrier();  // the state entering chunk n is in LDS
+#pragma unroll
+      for (int p = 0; p < 4; ++p) *reinterpret_cast<u32x4*>(&ks[16 * p + kr][kc]) = x.k[p];
+      if (n * GC + GC > T)  // rows past T (a sequence's last chunk): zeros
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+          if (n * GC + 16 * p + kr >= T) *reinterpret_cast<u32x4*>(&ks[16 * p + kr][kc]) = u32x4{0u, 0u, 0u, 0u};
+      const float el = __expf(x.last);
+      put_q(x, n + 1);
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const float av[4] = {x.a[p][0], x.a[p][1], x.a[p][2], x.a[p][3]};
+        store_hi_lo4(&ah[er + 16 * p][4 * ec], &al[er + 16 * p][4 * ec], av);
+      }
+      load_k(x, min(n + 2, N - 1));
+      load_a(x, min(n + 2, N - 1));
+      load_q(x, min(n + 3, N - 1));
+      if (h_chunks)  // the state entering chunk n, for the backward
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          h_chunks[((bh * N + n) * GD + rb + 8 * (r / 4) + 4 * lh + r % 4) * GD + cb + lc] = acc[r];
-    }
-    __syncthreads();
-    const bool more = n + 1 < N;
-    if (wave >= 4 && more) fetch(n + 1);
-    if (wave < 4) {  // w S (waves 0-1) or (q scale) S (waves 2-3), K = 128
-      const bf16_t* P = wave < 2 ? &ws[0][0] : &qs[0][0];
-      acc = f32x16{};
-      f32x16 acc2 = {};
-      bf16x8 pf[2], fh[2], fl[2];
-      auto frags = [&](int s, int k0) {
-        const int kk = k0 + 8 * lh;
-        pf[s] = frag_row<GP>(P, rb + lc, kk);
-        fh[s] = frag_row<GP>(&shh[0][0], lc, kk);
-        fl[s] = frag_row<GP>(&shl[0][0], lc, kk);
-      };
-      frags(0, 0);
+          (h_chunks + ((bh * N + n) * GD + 8 * (r / 4) + r % 4) * GD)[(uint32_t)(rb + 4 * lh) * GD + cb + lc] = acc[r];
+      bf16x8 pf[GC / 16];  // k^T of all four steps
 #pragma unroll
-      for (int j = 0; j < GD / 16; ++j) {
-        if (j + 1 < GD / 16) frags((j + 1) & 1, 16 * (j + 1));
-        __builtin_amdgcn_sched_barrier(0);
-        acc = mma_bf16(pf[j & 1], fh[j & 1], acc);
-        acc2 = mma_bf16(pf[j & 1], fl[j & 1], acc2);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[r] += acc2[r];
-      if (wave < 2) {  // v_new = u - w S, to LDS as hi / lo and, scaled by exp(gcum_last - gcum), for the update
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          const int t = rb + 8 * q4 + 4 * lh;
-          float vv[4], vk[4];
-#pragma unroll
-          for (int x = 0; x < 4; ++x) {
-            vv[x] = bf16_to_f32(us[t + x][lc]) - acc[4 * q4 + x];
-            vk[x] = vv[x] * ek[t + x];
-          }
-          store_hi_lo4(&vh[lc][t], &vl[lc][t], vv);
-          store_hi_lo4(&vkh[lc][t], &vkl[lc][t], vk);
-        }
-      } else {  // inter = (q S) e^gcum
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[r] *= __expf(gc[rb + 8 * (r / 4) + 4 * lh + r % 4]);
-        if (more) fetch(n + 1);
-      }
-    }
-    __syncthreads();  // v_new is in LDS
-    if (wave < 2) {
-      if (more) fetch(n + 1);
-    } else if (wave < 4) {  // o = inter + attn v_new (attn is zero above the diagonal), K = 64
-      bf16x8 ph[2], pl[2], qh[2], ql[2];
-      auto frags = [&](int s, int k0) {
-        const int kk = k0 + 8 * lh;
-        ph[s] = frag_row<KP>(&ah[0][0], rb + lc, kk);
-        pl[s] = frag_row<KP>(&al[0][0], rb + lc, kk);
-        qh[s] = frag_row<KP>(&vh[0][0], lc, kk);
-        ql[s] = frag_row<KP>(&vl[0][0], lc, kk);
-      };
-      frags(0, 0);
-      f32x16 acc2 = {};
-#pragma unroll
-      for (int j = 0; j < GC / 16; ++j) {
-        if (j + 1 < GC / 16) frags((j + 1) & 1, 16 * (j + 1));
-        __builtin_amdgcn_sched_barrier(0);
-        acc = mma_bf16(ph[j & 1], qh[j & 1], acc);
-        acc2 = mma_bf16(ph[j & 1], ql[j & 1], acc2);
-        acc2 = mma_bf16(pl[j & 1], qh[j & 1], acc2);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[r] += acc2[r];
-      if (o)  // the backward's recompute needs the states only
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int t = rb + 8 * (r / 4) + 4 * lh + r % 4;
-          if (t0 + t < T) o[((row0 + t0 + t) * H + h) * GD + cb + lc] = f32_to_bf16(acc[r]);
-        }
-    } else {  // S = e^gcum_last S + k^T (e^(gcum_last - gcum) v_new), K = 64
-      const float el = __expf(gc[GC - 1]);
+      for (int j = 0; j < GC / 16; ++j) pf[j] = frag_col<GP>(&ks[0][0], rb, 16 * j, lane);
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[r] *= el;
-      bf16x8 pf[2], fh[2], fl[2];
-      auto frags = [&](int s, int k0) {
-        const int kk = k0 + 8 * lh;
-        pf[s] = frag_col<GP>(&ks[0][0], rb, k0, lane);
-        fh[s] = frag_row<KP>(&vkh[0][0], lc, kk);
-        fl[s] = frag_row<KP>(&vkl[0][0], lc, kk);
-      };
-      frags(0, 0);
+      lds_barrier();  // v_new is in LDS
+      bf16x8 fh[GC / 16], fl[GC / 16];
+#pragma unroll
+      for (int j = 0; j < GC / 16; ++j) {
+        fh[j] = frag_row<KP>(&vkh[0][0], lc, 16 * j + 8 * lh);
+        fl[j] = frag_row<KP>(&vkl[0][0], lc, 16 * j + 8 * lh);
+      }
+      __builtin_amdgcn_sched_barrier(0);
       f32x16 acc2 = {};
 #pragma unroll
       for (int j = 0; j < GC / 16; ++j) {
-        if (j + 1 < GC / 16) frags((j + 1) & 1, 16 * (j + 1));
-        __builtin_amdgcn_sched_barrier(0);
-        acc = mma_bf16(pf[j & 1], fh[j & 1], acc);
-        acc2 = mma_bf16(pf[j & 1], fl[j & 1], acc2);
-        __builtin_amdgcn_sched_barrier(0);
+        acc = mma_bf16(pf[j], fh[j], acc);
+        acc2 = mma_bf16(pf[j], fl[j], acc2);
       }
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[r] += acc2[r];
-      if (more) put_state();  // phase B of this chunk, the last reader of shh / shl, is past the barrier
-    }
-  }
-  if (h_out && wave >= 4)
+      put_state();  // phase one of this chunk, the last reader of shh / shl, is past the barrier
+    };
+    load_q(sets[1], 0);
+    load_k(sets[0], 0);
+    load_a(sets[0], 0);
+    load_q(sets[0], min(1, N - 1));
+    put_q(sets[1], 0);
+    load_k(sets[1], min(1, N - 1));
+    load_a(sets[1], min(1, N - 1));
+    load_q(sets[1], min(2, N - 1));
+    put_state();
+    all_chunks(sets, chunk);
+    if (h_out)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int d = rb + 8 * (r / 4) + 4 * lh + r % 4;
-      h_out[(bh * GD + d) * GD + cb + lc] = acc[r];
-    }
+      for (int r = 0; r < 16; ++r)
+        h_out[(bh * GD + rb + 8 * (r / 4) + 4 * lh + r % 4) * GD + cb + lc] = acc[r];
+  }
 }
 
 
