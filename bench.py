@@ -868,8 +868,8 @@ def ragged_bench(a):
         res[name] = dict(fwd_ms=round(tf, 4), fwd_TFs=round(fl / (tf * 1e-3) / 1e12, 1), bwd_ms=round(tb, 4),
                          bwd_TFs=round(2 * fl / (tb * 1e-3) / 1e12, 1),
                          hipblaslt_dense_same_shape_TFs=round(fl / (th * 1e-3) / 1e12, 1))
-    # f32 operands at the up shape: three bf16 terms per value, six term products (a GEMM six times as deep) plus the
-    # split kernels; TF/s count the f32 product's 2 M K N, against the fp32 matrix peak
+    # f32 operands at the up shape: three bf16 terms per value, six term products;
+    # TF/s count the f32 product's 2 M K N, against the fp32 matrix peak
     K, Nn = 1024, 512
     lhs = torch.randn((M, K), device=dev, generator=gen)
     rhs = torch.randn((E, K, Nn), device=dev, generator=gen) * 0.02

@@ -5,6 +5,7 @@
 
 #include "chunk_table.h"
 #include "gemm256.h"
+#include "gemm_f32.h"
 #include "gemm_kernels.h"
 #include "launchers.h"
 
@@ -198,50 +199,6 @@ __global__ void zero_rows_from_kernel(void* __restrict__ out, int64_t m, int64_t
     if (esize == 4) ((float*)out)[r0 * n + x] = 0.f;
     else ((bf16_t*)out)[r0 * n + x] = 0;
   }
-}
-
-// f32 operands on the bf16 matrix cores.  An f32 value x is the sum of three bf16 terms x0 = bf16(x),
-// x1 = bf16(x - x0), x2 = bf16(x - x0 - x1) (round to nearest even; each difference is exact in f32): 24 significant
-// bits.  The product x y is the sum of the six term products of order <= 2 (x0 y0, x1 y0, x2 y0, x0 y1, x1 y1,
-// x0 y2); the three left out and the remainder of each split are below 2^-24 |x y|, and every term product is exact
-// in the MFMA's f32 accumulation.  Laid side by side along a GEMM's reduction dimension, the six products are one
-// bf16 GEMM of six times the depth.  Term j of a split row is term ((pattern >> 2j) & 3) of the f32 row; the two
-// patterns below pair up as (t_j, s_j) = (0,0) (1,0) (2,0) (0,1) (1,1) (0,2).
-constexpr uint32_t kSplitT = 0u | 1u << 2 | 2u << 4 | 0u << 6 | 1u << 8 | 0u << 10;  // terms 0 1 2 0 1 0
-constexpr uint32_t kSplitS = 0u | 0u << 2 | 0u << 4 | 1u << 6 | 1u << 8 | 2u << 10;  // terms 0 0 0 1 1 2
-
-// x [rows, cols] f32 -> out [rows, 6 cols] bf16: out[r, j cols + c] = term ((PAT >> 2j) & 3) of x[r, c].  cols % 4 == 0
-// and x 16-byte aligned; one float4 per lane and step, six 8-byte stores (HBM-bound: 4 bytes in, 12 out per value).
-template <uint32_t PAT>
-__global__ __launch_bounds__(256) void split3_bf16_kernel(const float* __restrict__ x, int64_t rows, int64_t cols,
-                                                          bf16_t* __restrict__ out) {
-  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-  const int64_t c4n = cols / 4;
-  for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
-    const float4* __restrict__ xr = reinterpret_cast<const float4*>(x + r * cols);
-    bf16_t* __restrict__ orow = out + r * 6 * cols;
-    for (int64_t c4 = (int64_t)blockIdx.x * 256 + threadIdx.x; c4 < c4n; c4 += (int64_t)gridDim.x * 256) {
-      const float4 v = xr[c4];
-      float rem[4] = {v.x, v.y, v.z, v.w};
-      u32x2 t[3];
-#pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        t[q] = u32x2{pack_bf16x2(rem[0], rem[1]), pack_bf16x2(rem[2], rem[3])};
-        rem[0] -= __uint_as_float(t[q][0] << 16);
-        rem[1] -= __uint_as_float(t[q][0] & 0xffff0000u);
-        rem[2] -= __uint_as_float(t[q][1] << 16);
-        rem[3] -= __uint_as_float(t[q][1] & 0xffff0000u);
-      }
-#pragma unroll
-      for (int j = 0; j < 6; ++j)
-        *reinterpret_cast<u32x2*>(orow + j * cols + 4 * c4) = t[(PAT >> (2 * j)) & 3];
-    }
-  }
-}
-
-// group sizes times f (the row counts of the split weight gradient)
-__global__ void scale_counts_kernel(const int32_t* __restrict__ gs, int e, int f, int32_t* __restrict__ out) {
-  for (int i = threadIdx.x; i < e; i += blockDim.x) out[i] = gs[i] * f;
 }
 
 inline unsigned pad8(int64_t g) { return (unsigned)((g + 7) / 8 * 8); }
@@ -590,14 +547,14 @@ int gemm_wgrad(int kid, int E, const int32_t* e_row0, int row0_mult, const int32
   return LSURGE_OK;
 }
 
-WgradChunkPlan wgrad_chunk_plan(int64_t M, int64_t E) {
+WgradChunkPlan wgrad_chunk_plan(int64_t M, int64_t E, int64_t min_rows) {
   WgradChunkPlan p;
-  // R: at least 2048 rows and 1.5 x the mean expert load, so balanced routings keep one chunk per routed expert,
+  // R: at least min_rows (2048) rows and 1.5 x the mean expert load, so balanced routings keep one chunk per routed expert,
   // while a hot expert (or the shared expert's rows) is cut into chunks near the routed ones' size, which keeps the
   // XCDs' shares of the launch even.  (A floor of M / 32 rows made C2's shared-expert chunks 3584 rows against
   // 1536-row routed ones; without it the C2 / C3 weight gradients run 1-7% faster.)  At most 2 M / R partial slots.
   const int64_t mean15 = ((3 * M + 2 * E - 1) / (2 * E) + BM - 1) / BM * BM;  // 1.5 x the mean load, in blocks
-  p.R = (int)std::max<int64_t>(2048, mean15);
+  p.R = (int)std::max<int64_t>(min_rows, mean15);
   p.max_chunks = (int)(E + (M + p.R - 1) / p.R);
   p.max_parts = (int)std::max<int64_t>(1, (2 * M + p.R - 1) / p.R);
   return p;
@@ -877,47 +834,50 @@ static int ragged_setup(const int32_t* gs, int64_t m, int64_t e, void* ws, size_
 // row tiles of the bf16 / f16 ragged_dot GEMMs: 256 rows for the persistent kernel, else 128
 static int ragged_tile_rows() { return lsurge::gemm_variant() == LSURGE_GEMM_G256 ? 256 : 128; }
 
-// ---- f32 operands: three bf16 terms per value, six term products along a reduction six times as deep (the pairing
-// is described at split3_bf16_kernel).
-//   forward  out = A' B'      A' [m, 6k] = lhs terms t, B'_e [6k, n] = rhs terms s stacked along k
-//   dlhs     dl = G' R''^T    G' [m, 6n] = g terms s,   R''_e [k, 6n] = rhs terms t side by side along n
-//   drhs     dr_e = A'_e^T G'_e over 6 gs_e rows: A' and G' read as [6m, k] and [6m, n], whose row 6i + j holds term
-//            t_j of lhs row i and term s_j of g row i, so group e owns rows [6 start_e, 6 (start_e + gs_e))
+// ---- f32 operands: the kernels of gemm_f32.h over 256-row tiles
 static size_t al256(size_t b) { return (b + 255) / 256 * 256; }
-static size_t split_bytes(int64_t rows, int64_t cols) { return al256(12 * (size_t)std::max<int64_t>(0, rows) * cols); }
 
 size_t lsurge_ragged_dot_f32_workspace_bytes(int64_t m, int64_t kdim, int64_t n, int64_t e) {
-  return al256(lsurge_ragged_dot_workspace_bytes(m, e)) + split_bytes(m, kdim) + split_bytes(e * kdim, n);
+  return al256(lsurge_ragged_dot_workspace_bytes(m, e));
 }
 
-// the f32 backward's chunked weight gradient (e <= 256) runs over 6 m rows
-static bool f32_bwd_chunked(int64_t m, int64_t e) { return m > 0 && ragged_chunked(e); }
+// a row costs six products, so the chunks of the weight gradient are cut at a sixth of the 16-bit floor of rows
+static lsurge::WgradChunkPlan f32_chunk_plan(int64_t m, int64_t e) { return lsurge::wgrad_chunk_plan(m, e, 384); }
 
 size_t lsurge_ragged_dot_bwd_f32_workspace_bytes(int64_t m, int64_t kdim, int64_t n, int64_t e) {
-  size_t b = al256(lsurge_ragged_dot_workspace_bytes(m, e)) + al256(lsurge_ragged_dot_workspace_bytes(6 * m, e)) +
-             al256(sizeof(int32_t) * (size_t)std::max<int64_t>(e, 0)) + split_bytes(m, kdim) + split_bytes(m, n) +
-             split_bytes(e * kdim, n);
-  if (f32_bwd_chunked(m, e)) {
-    const lsurge::WgradChunkPlan p = lsurge::wgrad_chunk_plan(6 * m, e);
+  size_t b = al256(lsurge_ragged_dot_workspace_bytes(m, e));
+  if (m > 0 && ragged_chunked(e)) {
+    const lsurge::WgradChunkPlan p = f32_chunk_plan(m, e);
     b += al256(sizeof(int32_t) * lsurge::wgrad_chunk_table_ints(p, e)) + lsurge::wgrad_chunked_workspace_bytes(p, kdim, n);
   }
   return b;
 }
 
-// x [rows, cols] f32 -> [rows, 6 cols] bf16 terms in the order of pattern kSplitT (t) or kSplitS (s)
-static int split3(const float* x, int64_t rows, int64_t cols, bool t_terms, bf16_t* out, hipStream_t s) {
-  LSURGE_REQUIRE(cols % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)out % 16 == 0,
-                 "ragged_dot f32: operands must be 16-byte aligned with rows of a multiple of 4 values");
-  if (rows == 0) return LSURGE_OK;
-  const int64_t c4 = cols / 4;
-  const unsigned gx = (unsigned)std::min<int64_t>((c4 + 255) / 256, 1024);
-  const unsigned gy = (unsigned)std::min<int64_t>(rows, std::max<int64_t>(1, 8192 / gx));
-  if (t_terms)
-    LSURGE_LAUNCH(KID_MISC, s, hipLaunchKernelGGL(split3_bf16_kernel<kSplitT>, dim3(gx, gy), dim3(256), 0, s, x, rows,
-                                                  cols, out));
-  else
-    LSURGE_LAUNCH(KID_MISC, s, hipLaunchKernelGGL(split3_bf16_kernel<kSplitS>, dim3(gx, gy), dim3(256), 0, s, x, rows,
-                                                  cols, out));
+// spans are limited to 2 GiB counted at 12 bytes a value (the six bf16 terms of a product)
+static int check_f32(const void* p, int64_t span, const char* what) {
+  LSURGE_REQUIRE((uintptr_t)p % 16 == 0, "%s: operands must be 16-byte aligned", what);
+  return lsurge::check_desc(12 * span, what);
+}
+
+// C[rows, N] = A[rows, K] @ B_e over the 256-row tiles of g (nk: B_e stored [N, K]); f32 operands, f32 or bf16 C
+static int gemm_rows_f32(const lsurge::GemmBlocks& g, const float* A, const float* B, bool nk, int64_t K, int64_t N,
+                         void* C, bool out_f32, hipStream_t s, const char* what) {
+  if (int rc = check_f32(A, g.tile_rows * K, what)) return rc;
+  if (int rc = check_f32(B, K * N, what)) return rc;
+  if (int rc = lsurge::check_desc((int64_t)f32x3::BM * N * (out_f32 ? 4 : 2), what)) return rc;
+  RowsArgs a{};
+  a.A = (const bf16_t*)A; a.lda = K; a.B = (const bf16_t*)B; a.ldb = nk ? K : N; a.b_estride = K * N;
+  a.K = K; a.N = N; a.ldc = N;
+  if (out_f32) a.Cf = (float*)C;
+  else a.C = (bf16_t*)C;
+  a.t_expert = g.blk_expert; a.t_rows = g.blk_rows; a.t_row0 = g.blk_row0; a.num_tiles = g.num_blocks;
+  a.max_tiles = g.max_blocks;
+  a.n_tiles = (int)((N + f32x3::BN - 1) / f32x3::BN);
+  if (a.max_tiles == 0) return LSURGE_OK;
+  const dim3 grid(f32x3::NWG), block(256);
+  if (nk) LSURGE_LAUNCH(KID_MISC, s, hipLaunchKernelGGL((f32x3::rows_kernel<B_NK, false>), grid, block, 0, s, a));
+  else if (out_f32) LSURGE_LAUNCH(KID_MISC, s, hipLaunchKernelGGL((f32x3::rows_kernel<B_KN, false>), grid, block, 0, s, a));
+  else LSURGE_LAUNCH(KID_MISC, s, hipLaunchKernelGGL((f32x3::rows_kernel<B_KN, true>), grid, block, 0, s, a));
   return LSURGE_OK;
 }
 
@@ -928,20 +888,12 @@ static int ragged_dot_f32(const float* lhs, const float* rhs, const int32_t* gs,
   if (int rc = lsurge::check_gemm_shape(kdim, n, "ragged_dot f32")) return rc;
   const size_t need = lsurge_ragged_dot_f32_workspace_bytes(m, kdim, n, e);
   LSURGE_REQUIRE(ws && ws_bytes >= need, "ragged_dot f32: workspace %zu < %zu bytes", ws_bytes, need);
-  char* base = (char*)ws;
-  size_t off = al256(lsurge_ragged_dot_workspace_bytes(m, e));
-  bf16_t* a2 = (bf16_t*)(base + off);
-  off += split_bytes(m, kdim);
-  bf16_t* b2 = (bf16_t*)(base + off);
+  LSURGE_REQUIRE((uintptr_t)ws % 16 == 0, "ragged_dot f32: workspace must be 16-byte aligned");
   lsurge::GemmBlocks g;
   int32_t *total, *e_row0, *e_rows;
-  if (int rc = ragged_setup(gs, m, e, ws, ws_bytes, s, &g, &total, &e_row0, &e_rows, ragged_tile_rows())) return rc;
-  if (int rc = split3(lhs, m, kdim, true, a2, s)) return rc;
-  if (int rc = split3(rhs, e, kdim * n, false, b2, s)) return rc;
+  if (int rc = ragged_setup(gs, m, e, ws, ws_bytes, s, &g, &total, &e_row0, &e_rows, f32x3::BM)) return rc;
   const bool f32 = out_dtype == LSURGE_F32;
-  if (int rc = lsurge::gemm_rows_kn(KID_MISC, g, a2, 6 * kdim, b2, n, 6 * kdim * n, 6 * kdim, n, out, n, s, f32,
-                                    lsurge::ExtraExpert(), LSURGE_BF16))
-    return rc;
+  if (int rc = gemm_rows_f32(g, lhs, rhs, false, kdim, n, out, f32, s, "ragged_dot f32")) return rc;
   LSURGE_LAUNCH(KID_MISC, s,
                 hipLaunchKernelGGL(zero_rows_from_kernel, dim3(1024), dim3(256), 0, s, out, m, n, f32 ? 4 : 2, total));
   return LSURGE_OK;
@@ -950,48 +902,51 @@ static int ragged_dot_f32(const float* lhs, const float* rhs, const int32_t* gs,
 static int ragged_dot_bwd_f32(const float* lhs, const float* rhs, const int32_t* gs, const float* g, int64_t m,
                               int64_t kdim, int64_t n, int64_t e, float* dlhs, float* drhs, void* ws, size_t ws_bytes,
                               hipStream_t s) {
-  if (int rc = lsurge::check_gemm_shape(kdim, n, "ragged_dot_bwd f32")) return rc;
-  LSURGE_REQUIRE(6 * m < (1ll << 31), "ragged_dot_bwd f32: m=%lld too large (6 m rows)", (long long)m);
+  const char* what = "ragged_dot_bwd f32";
+  if (int rc = lsurge::check_gemm_shape(kdim, n, what)) return rc;
   const size_t need = lsurge_ragged_dot_bwd_f32_workspace_bytes(m, kdim, n, e);
   LSURGE_REQUIRE(ws && ws_bytes >= need, "ragged_dot_bwd f32: workspace %zu < %zu bytes", ws_bytes, need);
+  LSURGE_REQUIRE((uintptr_t)ws % 16 == 0, "ragged_dot_bwd f32: workspace must be 16-byte aligned");
+  if (int rc = check_f32(lhs, m * kdim, what)) return rc;
+  if (int rc = check_f32(g, m * n, what)) return rc;
   char* base = (char*)ws;
-  const size_t t1 = al256(lsurge_ragged_dot_workspace_bytes(m, e));
-  const size_t t6 = al256(lsurge_ragged_dot_workspace_bytes(6 * m, e));
-  int32_t* gs6 = (int32_t*)(base + t1 + t6);
-  size_t off = t1 + t6 + al256(sizeof(int32_t) * e);
-  bf16_t* a2 = (bf16_t*)(base + off);
-  off += split_bytes(m, kdim);
-  bf16_t* g2 = (bf16_t*)(base + off);
-  off += split_bytes(m, n);
-  bf16_t* r2 = (bf16_t*)(base + off);
-  off += split_bytes(e * kdim, n);
-  lsurge::GemmBlocks gb, gb6;
-  int32_t *total, *e_row0, *e_rows, *total6, *e_row0_6, *e_rows_6;
-  if (int rc = ragged_setup(gs, m, e, base, t1, s, &gb, &total, &e_row0, &e_rows, ragged_tile_rows())) return rc;
-  LSURGE_LAUNCH(KID_MISC, s, hipLaunchKernelGGL(scale_counts_kernel, dim3(1), dim3(256), 0, s, gs, (int)e, 6, gs6));
-  if (int rc = ragged_setup(gs6, 6 * m, e, base + t1, t6, s, &gb6, &total6, &e_row0_6, &e_rows_6)) return rc;
-  if (int rc = split3(lhs, m, kdim, true, a2, s)) return rc;
-  if (int rc = split3(g, m, n, false, g2, s)) return rc;
-  if (int rc = split3(rhs, e * kdim, n, true, r2, s)) return rc;
+  lsurge::GemmBlocks gb;
+  int32_t *total, *e_row0, *e_rows;
+  if (int rc = ragged_setup(gs, m, e, base, ws_bytes, s, &gb, &total, &e_row0, &e_rows, f32x3::BM)) return rc;
   if (m > 0) {
-    if (int rc = lsurge::gemm_rows_nk(KID_MISC, gb, g2, 6 * n, r2, nullptr, 0, 6 * n, 6 * kdim * n, 6 * n, kdim, dlhs,
-                                      kdim, false, nullptr, nullptr, 0, s, true, lsurge::ExtraExpert(), LSURGE_BF16))
-      return rc;
+    if (int rc = gemm_rows_f32(gb, g, rhs, true, n, kdim, dlhs, true, s, what)) return rc;
     LSURGE_LAUNCH(KID_MISC, s,
                   hipLaunchKernelGGL(zero_rows_from_kernel, dim3(1024), dim3(256), 0, s, dlhs, m, kdim, 4, total));
   }
-  if (f32_bwd_chunked(m, e)) {
-    const lsurge::WgradChunkPlan p = lsurge::wgrad_chunk_plan(6 * m, e);
+  // drhs: the groups' rows in chunks that spread a hot group over the GPU (e <= 256), else one slice per group
+  WgradArgs a{};
+  a.A = (const bf16_t*)lhs; a.lda = kdim; a.B = (const bf16_t*)g; a.ldb = n; a.I = kdim; a.N = n; a.C = drhs; a.ldc = n;
+  a.c_estride = kdim * n; a.E = (int)e;
+  a.e_row0 = e_row0; a.e_rows = e_rows;
+  a.i_tiles = (int)((kdim + f32x3::BM - 1) / f32x3::BM);
+  a.n_tiles = (int)((n + f32x3::BN - 1) / f32x3::BN);
+  const bool chunked = m > 0 && ragged_chunked(e);
+  lsurge::WgradChunks ch;
+  if (chunked) {
+    const lsurge::WgradChunkPlan p = f32_chunk_plan(m, e);
+    size_t off = al256(lsurge_ragged_dot_workspace_bytes(m, e));
     int32_t* table = (int32_t*)(base + off);
     off += al256(sizeof(int32_t) * lsurge::wgrad_chunk_table_ints(p, e));
-    lsurge::WgradChunks ch;
-    if (int rc = lsurge::build_wgrad_chunks(e_rows_6, e_row0_6, (int)e, p, table, &ch, s, -1, 0, 1)) return rc;
-    return lsurge::gemm_wgrad_chunked(KID_MISC, ch, (int)e, 6 * m, a2, kdim, g2, n, kdim, n, drhs, nullptr, 0, n,
-                                      kdim * n, base + off, lsurge::wgrad_chunked_workspace_bytes(p, kdim, n), s,
-                                      lsurge::RowGather(), lsurge::ExtraOut(), LSURGE_BF16);
+    if (int rc = lsurge::build_wgrad_chunks(e_rows, e_row0, (int)e, p, table, &ch, s, -1, 0, 1)) return rc;
+    a.part = (float*)(base + off);
+    a.c_expert = ch.c_expert; a.c_row0 = ch.c_row0; a.c_rows = ch.c_rows; a.c_part = ch.c_part;
+    a.num_chunks = ch.num_chunks; a.max_chunks = ch.max_chunks;
   }
-  return lsurge::gemm_wgrad(KID_MISC, (int)e, e_row0_6, 1, e_rows_6, 0, 6 * m, a2, kdim, g2, n, kdim, n, drhs, nullptr,
-                            0, n, kdim * n, 1, nullptr, 0, s, lsurge::RowGather(), LSURGE_BF16);
+  LSURGE_LAUNCH(KID_MISC, s, hipLaunchKernelGGL((f32x3::wgrad_kernel<>), dim3(f32x3::NWG), dim3(256), 0, s, a));
+  if (chunked) {
+    const unsigned grid = (unsigned)std::min<int64_t>(2 * ((kdim * n / 4 + 255) / 256), 2048);
+    LSURGE_LAUNCH(KID_SPLITK_REDUCE, s,
+                  hipLaunchKernelGGL(wgrad_chunk_reduce_kernel, dim3(grid), dim3(256), 0, s, (const float*)a.part,
+                                     ch.split_list, ch.num_split, ch.e_pbase, ch.e_nparts, kdim, n, drhs,
+                                     (float*)nullptr, (int64_t)0, n, kdim * n, -1, (float*)nullptr, (float*)nullptr,
+                                     (int)LSURGE_F32));
+  }
+  return LSURGE_OK;
 }
 
 int lsurge_ragged_dot(const void* lhs, const void* rhs, const int32_t* group_sizes, int64_t m, int64_t kdim, int64_t n,
@@ -1150,8 +1105,7 @@ int lsurge_ragged_dot_noalloc(const void* lhs, const void* rhs, const int32_t* g
   LSURGE_REQUIRE(need <= sizeof(int32_t) * kScratchInts, "ragged_dot_noalloc: table of %zu bytes exceeds the scratch",
                  need);
   if (in_dtype == LSURGE_F32)
-    return lsurge::set_error(LSURGE_ERR_DTYPE, "ragged_dot_noalloc: f32 operands need the split-term workspace of "
-                             "lsurge_ragged_dot");
+    return lsurge::set_error(LSURGE_ERR_DTYPE, "ragged_dot_noalloc: f32 operands are lsurge_ragged_dot's");
   if (m == 0) return LSURGE_OK;
   int32_t* ws = scratch_on_current_device();
   if (!ws) return LSURGE_ERR_LAUNCH;

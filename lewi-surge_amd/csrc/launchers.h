@@ -150,7 +150,7 @@ struct WgradChunks {
   const int32_t *c_expert, *c_row0, *c_rows, *c_part, *num_chunks, *e_pbase, *e_nparts, *split_list, *num_split;
   int max_chunks, max_parts;
 };
-WgradChunkPlan wgrad_chunk_plan(int64_t M, int64_t E);
+WgradChunkPlan wgrad_chunk_plan(int64_t M, int64_t E, int64_t min_rows = 2048);
 // A dense weight gradient C[I, N] = A^T B over M rows as the chunk table's only (extra) expert: ceil(256 / tiles of
 // 256 x 256) chunks of equal rows (at most 16, at least 1024 rows each), so the chunks' tiles fill the GPU once.
 WgradChunkPlan wgrad_chunk_plan_dense(int64_t M, int64_t I, int64_t N);

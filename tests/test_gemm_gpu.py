@@ -139,6 +139,21 @@ def test_f32_operands_many_groups(dev):
     assert max(errs) <= F32_TOL, errs
 
 
+@pytest.mark.parametrize("gs,tail,K,N", [
+    ([1, 0, 255, 256, 257], 1, 8, 8),            # one 16-deep stage (and its zero partner), one narrow column tile
+    ([15, 16, 17, 33, 31], 0, 40, 264),          # row remainders of a weight-gradient stage, a second tile of 8 columns
+    ([3, 511, 0, 2], 300, 264, 40),              # a second tile of 8 gradient rows; tail rows outside every group
+    ([1500, 5], 0, 272, 520),                    # a group cut into several weight-gradient chunks
+    ([0] * 40 + [1], 0, 128, 128),               # fewer tiles than XCDs, empty groups' zero gradients
+    ([2] * 290, 3, 48, 280),                     # more than 256 groups: one slice a group
+])
+def test_f32_operands_tile_edges(gs, tail, K, N, dev):
+    """The f32 kernels' 256 x 256 x 16 stages at their edges.  Terms left out and split remainders stay below 2^-22 of
+    the products and f32 accumulation below sqrt(depth) 2^-24, far inside the reference's f32 tolerance."""
+    errs = run_case_f32(gs, sum(gs) + tail, K, N, dev, seed=K + N)
+    assert max(errs) <= F32_TOL, errs
+
+
 def test_f32_operands_unaligned_and_bf16_out(dev):
     """lhs / rhs starting 4 bytes into their storage (copied to aligned memory first), and bf16 output of f32
     operands (the output rounding bounds the forward; the gradients stay f32)."""
