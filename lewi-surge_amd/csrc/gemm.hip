@@ -831,8 +831,14 @@ static int ragged_setup(const int32_t* gs, int64_t m, int64_t e, void* ws, size_
   return LSURGE_OK;
 }
 
-// row tiles of the bf16 / f16 ragged_dot GEMMs: 256 rows for the persistent kernel, else 128
-static int ragged_tile_rows() { return lsurge::gemm_variant() == LSURGE_GEMM_G256 ? 256 : 128; }
+// row tiles of the bf16 / f16 ragged_dot GEMMs: 256 rows for the persistent kernel, else 128 (the 4-wave kernel).  With a
+// mean of at most 64 rows a group the weights' read bounds the call, and the 4-wave kernel's two workgroups a CU keep
+// more of it in flight: K = 1024, N = 512, 128 groups of 7 / 64 rows, forward 47.4 / 51.0 -> 45.5 / 45.8 us, backward
+// 98 / 109 -> 94 / 101 us; 8 groups of K = 2048, 48.6 / 48.8 -> 41.4 / 45.2 us.  At 128 rows a group it is 3 us slower or
+// faster by the shape, at 256 rows it is up to 11 us slower.
+static int ragged_tile_rows(int64_t m, int64_t e) {
+  return lsurge::gemm_variant() == LSURGE_GEMM_G256 && m > 64 * e ? 256 : 128;
+}
 
 // ---- f32 operands: the kernels of gemm_f32.h over 256-row tiles
 static size_t al256(size_t b) { return (b + 255) / 256 * 256; }
@@ -969,7 +975,7 @@ int lsurge_ragged_dot(const void* lhs, const void* rhs, const int32_t* group_siz
   lsurge::GemmBlocks g;
   int32_t *total, *e_row0, *e_rows;
   if (int rc = ragged_setup(group_sizes, m, e, workspace, workspace_bytes, s, &g, &total, &e_row0, &e_rows,
-                            ragged_tile_rows()))
+                            ragged_tile_rows(m, e)))
     return rc;
   const bool f32 = out_dtype == LSURGE_F32;
   if (int rc = lsurge::gemm_rows_kn(KID_MISC, g, lhs, kdim, rhs, n, kdim * n, kdim, n, out, n, s, f32,
@@ -1159,7 +1165,7 @@ int lsurge_ragged_dot_bwd_as(const void* lhs, const void* rhs, const int32_t* gr
   lsurge::GemmBlocks gb;
   int32_t *total, *e_row0, *e_rows;
   if (int rc = ragged_setup(group_sizes, m, e, workspace, workspace_bytes, s, &gb, &total, &e_row0, &e_rows,
-                            ragged_tile_rows()))
+                            ragged_tile_rows(m, e)))
     return rc;
   // dlhs[r] = g[r] @ rhs[e]^T : rhs[e] is [K, N] = k-major storage of the [N -> K] operand
   if (m > 0) {

@@ -469,9 +469,16 @@ static int moe_fwd_impl(const lsurge_moe_shape* s, const lsurge_moe_params* p, c
   // C2, measured with the vector-unit router before this one: 1.547 -> 1.537 ms per step (same-box A/B against forking
   // after the router with the persistent kernels).
   const bool early = !w8 && q.fs && s0 != st;
+  // Few rows per expert (a mean of at most one 128-row block): the routed GEMMs are bound by the weights' read, and the
+  // 4-wave kernel on 128-row blocks keeps two workgroups and twice the copies in flight on a CU, where the persistent
+  // kernel's 256-row tiles give every CU one or two tiles (at 64 experts and d = 1024 the shared expert's four are a
+  // second round for four CUs).  Forward, 64 experts, k = 6, cold weights: T = 64 146 -> 131 us, 1024 150 -> 143; 128
+  // experts, T = 512 200 -> 182.  From two blocks an expert on the persistent kernel's tiles fill: T = 4096, 64 experts
+  // 198 against 219 us.  Both kernels give the same bits.
+  const bool few = !w8 && q.M <= BLK * q.E;
   // a merged shared expert forked early: its down projection rides along the routed down GEMM as expert E (its
   // tiles follow the routed ones in the tile table), so the helper's classic-kernel GEMMs end with the layout
-  const bool ride = early && q.merged && lsurge::gemm_variant() == LSURGE_GEMM_G256;
+  const bool ride = early && q.merged && !few && lsurge::gemm_variant() == LSURGE_GEMM_G256;
   if (early)
     if (int rc = lsurge::stream_after(s0, st, fg.f.ev[3])) return rc;
   // W_r^T for the backward's router dx term (saved): on the helper stream when it forks here (off the critical path),
@@ -550,9 +557,9 @@ static int moe_fwd_impl(const lsurge_moe_shape* s, const lsurge_moe_params* p, c
                                          (char*)workspace + hist_bytes + f8_bytes,
                                          workspace_bytes - hist_bytes - f8_bytes, st, tiles, chunks))
     return rc;
-  // the routed forward GEMMs: the 256-row tiles (routed ones) on the persistent kernel, or, with the classic kernels,
-  // 128-row blocks on the 4-wave kernel (the ping-pong kernel measured no faster there)
-  const lsurge::GemmBlocks blocks = lsurge::gemm_variant() == LSURGE_GEMM_G256
+  // the routed forward GEMMs: the 256-row tiles (routed ones) on the persistent kernel, or, with few rows per expert or
+  // the classic kernels, 128-row blocks on the 4-wave kernel (the ping-pong kernel measured no faster there)
+  const lsurge::GemmBlocks blocks = !few && lsurge::gemm_variant() == LSURGE_GEMM_G256
                                         ? lsurge::GemmBlocks{sv.t_expert, sv.t_rows, sv.t_row0, sv.num_tiles, (int)q.TB, 0, 256}
                                         : lsurge::GemmBlocks{sv.blk_expert, sv.blk_rows, nullptr, sv.num_blocks, (int)q.MB, 0};
   lsurge::RowGather gather;

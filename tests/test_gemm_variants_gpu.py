@@ -106,6 +106,34 @@ def test_layer_bitwise(T, d, E, k, f, fs, zipf, dev):
         assert torch.equal(x0, x1), f"{name}: max |diff| {(x0.float() - x1.float()).abs().max().item()}"
 
 
+@pytest.mark.parametrize("m,e,hot", [(256, 4, False), (257, 4, False), (512, 8, True), (513, 8, True), (64, 1, False)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_ragged_dot_few_rows_rule(m, e, hot, dt, dev):
+    """Both sides of the few-rows rule (m = 64 e rows and one more), all rows in one group included: the bits of the
+    classic kernels, forward and backward."""
+    gs = [0] * e
+    if hot:
+        gs[-1] = m
+    else:
+        gs = [m // e] * e
+        gs[0] += m % e
+    res = _ragged(gs, m, 72, 264, dt, None, dev, seed=m)
+    for x0, x1 in zip(res[0], res[1]):
+        assert torch.equal(x0, x1)
+
+
+@pytest.mark.parametrize("T", [512, 513])
+@pytest.mark.parametrize("fs", [0, 128, 256])
+@pytest.mark.parametrize("zipf", [False, True])
+def test_layer_few_rows_rule(T, fs, zipf, dev):
+    """Both sides of the layer's few-rows rule (T k = 128 E slots and k more), with the shared expert merged, of its own
+    width and absent: the bits of the classic kernels."""
+    p = mo.make_inputs(T=T, d=256, E=16, k=4, f=128, fs=fs, seed=T + fs, zipf=zipf)
+    res = _layer(p, MoEShape(T, 256, 16, 4, 128, fs), dev)
+    for name in res[0]:
+        assert torch.equal(res[0][name], res[1][name]), name
+
+
 @pytest.mark.parametrize("M,K,N,E,hot,dtype", [(1000, 64, 72, 8, 0, torch.bfloat16), (3000, 512, 520, 4, 2600, torch.bfloat16),
                                                (2304, 1024, 1024, 8, 0, torch.bfloat16), (700, 136, 256, 300, 0, torch.bfloat16),
                                                (9000, 256, 264, 2, 8900, torch.float16), (640, 128, 128, 8, 0, torch.float16)])
