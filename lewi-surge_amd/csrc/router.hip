@@ -290,13 +290,13 @@ __global__ __launch_bounds__(RL_THREADS) void router_logits_kernel(const bf16_t*
 // Logits.  v_mfma_f32_16x16x4_f32 adds its four products to the accumulator one after the other in ascending k, each
 // with one f32 rounding: exactly the fmaf chain of router_logits_kernel, at twice the vector unit's rate (measured
 // bit-equal on normal, wide-range, cancelling, subnormal and non-finite bf16 operands; the GPU tests compare the two
-// kernels bit for bit).  One workgroup = TOK = 16 TT tokens x all E experts, one wave per 32 experts; a wave holds TT
-// token tiles x 2 expert tiles (expert 32 wave + 2 c + h is column c of tile h, so one dword of a row of W_r feeds
-// both tiles).  Step s of a 32-deep block covers d = 4 s .. + 3, lane quarter q supplying d = 4 s + q:
+// kernels bit for bit).  One workgroup = TOK = 16 TT tokens x all E experts, one wave per 16 HT experts; a wave holds TT
+// token tiles x HT expert tiles (HT = 2: expert 32 wave + 2 c + h is column c of tile h, so one dword of a row of W_r
+// feeds both tiles).  Step s of a 32-deep block covers d = 4 s .. + 3, lane quarter q supplying d = 4 s + q:
 //   x  goes through a double LDS buffer of DC-deep chunks, each block of a row stored by quarter ([q][8 steps] bf16),
 //      so one 16-byte read gives a lane its operands of 8 steps; blocks are read one ahead of their use;
 //   w  straight from L2 into registers, a ring of GD / 4 steps ahead of its use.
-// Bound by the matrix pipe (64 cycles a step and token tile) once two waves share a SIMD, by load latency below that.
+// Bound by the matrix pipe (32 HT cycles a step and token tile) once two waves share a SIMD, by load latency below that.
 // TT = 1 gives the most workgroups, TT = 4 the fewest reads of W_r; the launcher takes the largest TT that still
 // leaves 2048 waves (two per SIMD), so small batches spread over the CUs and a 1 MB W_r is read once per 64 tokens.
 // At E = 256 the registers are held to 128, so that two 8-wave workgroups share a CU (656 -> 613 us at T = 65536, d =
@@ -308,8 +308,8 @@ __global__ __launch_bounds__(RL_THREADS) void router_logits_kernel(const bf16_t*
 //
 // Then, in the same workgroup:
 //  - the logits go to HBM and to an LDS tile [TOK][E + 1];
-//  - top-k + softmax per token: L = E / (8 TT) lanes per token each keep a sorted list of the best 8 of their
-//    EPL = 8 TT experts (scanned in ascending expert order, a logit moves ahead only of strictly smaller ones), and
+//  - top-k + softmax per token: L = E / (4 HT TT) lanes per token each keep a sorted list of the best 8 of their
+//    EPL = 4 HT TT experts (scanned in ascending expert order, a logit moves ahead only of strictly smaller ones), and
 //    k merge rounds take the best head of the L lists (larger logit, ties to the lower expert index) -- the order of
 //    a stable descending sort, as in router_select_lane_kernel, whose softmax (in rank order) this repeats;
 //  - the expert histogram of the workgroup's TOK k slots (LDS counters) -> hist[chunk of 64 tokens][E], the layout's
@@ -317,15 +317,15 @@ __global__ __launch_bounds__(RL_THREADS) void router_logits_kernel(const bf16_t*
 //    picks an expert at most once, so even 64 tokens fit one byte): a workgroup writes the TT bytes of its own
 //    quarters (its count and zeros), and the layout adds the four bytes up.  No workgroup touches another's bytes, so
 //    nothing has to be cleared first.
-template <int E, int TT, int DC>
-__global__ __launch_bounds__(2 * E, E == 256 ? 4 : 1) void router_fused_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+template <int E, int TT, int HT, int DC>
+__global__ __launch_bounds__(4 * E / HT, E == 256 ? 4 : 1) void router_fused_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                              const float* __restrict__ bias, int T, int d, int k,
                                                              float* __restrict__ logits, int32_t* __restrict__ sel,
                                                              float* __restrict__ weights, uint8_t* __restrict__ hist) {
-  constexpr int NT = 2 * E, TOK = 16 * TT, L = NT / TOK, EPL = E / L;  // threads, tokens, lanes and experts a lane
+  constexpr int NT = 4 * E / HT, TOK = 16 * TT, L = NT / TOK, EPL = E / L;  // threads, tokens, lanes and experts a lane
   constexpr int GD = DC < 128 ? DC : 128;    // depth of the weight ring
   constexpr int XP = 2 * DC + 16;            // LDS row pitch in bytes (rows one 16-byte slot apart in the banks)
-  static_assert(64 % L == 0 && L >= 1 && EPL >= 8, "fused router shape");
+  static_assert(64 % L == 0 && L >= 1 && (HT == 1 || HT == 2), "fused router shape");
   constexpr int XS_B = 2 * TOK * XP, TILE_B = TOK * (E + 1) * 4;
   __shared__ __attribute__((aligned(16))) char sm[XS_B > TILE_B ? XS_B : TILE_B];
   __shared__ int32_t cnt[E];
@@ -359,11 +359,16 @@ __global__ __launch_bounds__(2 * E, E == 256 ? 4 : 1) void router_fused_kernel(c
       }
     }
   };
-  const bf16_t* wl = w + (int64_t)q * E + 32 * wv + 2 * r;  // this lane's experts of d row q
-  auto gw = [&](int dd) { return *reinterpret_cast<const uint32_t*>(wl + (int64_t)dd * E); };
-  f32x4 acc[TT][2];
+  const bf16_t* wl = w + (int64_t)q * E + HT * (16 * wv + r);  // this lane's experts of d row q
+  auto gw = [&](int dd) {
+    if constexpr (HT == 2) return *reinterpret_cast<const uint32_t*>(wl + (int64_t)dd * E);
+    else return (uint32_t)wl[(int64_t)dd * E];
+  };
+  f32x4 acc[TT][HT];
 #pragma unroll
-  for (int a = 0; a < TT; ++a) acc[a][0] = acc[a][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int a = 0; a < TT; ++a)
+#pragma unroll
+    for (int h = 0; h < HT; ++h) acc[a][h] = f32x4{0.f, 0.f, 0.f, 0.f};
   uint32_t wr[GD / 4];
   gx(0);
 #pragma unroll
@@ -386,11 +391,11 @@ __global__ __launch_bounds__(2 * E, E == 256 ? 4 : 1) void router_fused_kernel(c
 #pragma unroll
       for (int b = 0; b < GD / 32; ++b) {
         fread(fa[(b + 1) & 1], min(g / 32 + b + 1, DC / 32 - 1));
-        float wc[8][2];
+        float wc[8][HT];
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
           wc[s][0] = __uint_as_float(wr[8 * b + s] << 16);
-          wc[s][1] = __uint_as_float(wr[8 * b + s] & 0xffff0000u);
+          if constexpr (HT == 2) wc[s][1] = __uint_as_float(wr[8 * b + s] & 0xffff0000u);
           wr[8 * b + s] = gw(dn + 32 * b + 4 * s);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -400,8 +405,8 @@ __global__ __launch_bounds__(2 * E, E == 256 ? 4 : 1) void router_fused_kernel(c
           for (int a = 0; a < TT; ++a) {
             const uint32_t u = fa[b & 1][a][s >> 1];
             const float xv = __uint_as_float(s & 1 ? u & 0xffff0000u : u << 16);
-            acc[a][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv, wc[s][0], acc[a][0], 0, 0, 0);
-            acc[a][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv, wc[s][1], acc[a][1], 0, 0, 0);
+#pragma unroll
+            for (int h = 0; h < HT; ++h) acc[a][h] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv, wc[s][h], acc[a][h], 0, 0, 0);
           }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -409,22 +414,28 @@ __global__ __launch_bounds__(2 * E, E == 256 ? 4 : 1) void router_fused_kernel(c
   }
   __syncthreads();  // every wave is done with the staging buffers: they now hold the logits tile
   float* lt = reinterpret_cast<float*>(sm);
-  const int e0 = 32 * wv + 2 * r;
-  const float b0 = bias ? bias[e0] : 0.f, b1 = bias ? bias[e0 + 1] : 0.f;
+  const int e0 = HT * (16 * wv + r);
+  float be[HT];
+#pragma unroll
+  for (int h = 0; h < HT; ++h) be[h] = bias ? bias[e0 + h] : 0.f;
 #pragma unroll
   for (int a = 0; a < TT; ++a)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {  // accumulator element i: token 4 q + i of the tile
       const int tt = 16 * a + 4 * q + i, t = t0 + tt;
-      const float v0 = bias ? acc[a][0][i] + b0 : acc[a][0][i], v1 = bias ? acc[a][1][i] + b1 : acc[a][1][i];
-      lt[tt * (E + 1) + e0] = v0;
-      lt[tt * (E + 1) + e0 + 1] = v1;
-      if (t < T) *reinterpret_cast<float2*>(logits + (int64_t)t * E + e0) = float2{v0, v1};
+      float v[HT];
+#pragma unroll
+      for (int h = 0; h < HT; ++h) lt[tt * (E + 1) + e0 + h] = v[h] = bias ? acc[a][h][i] + be[h] : acc[a][h][i];
+      if (t < T) {
+        float* lg = logits + (int64_t)t * E + e0;
+        if constexpr (HT == 2) *reinterpret_cast<float2*>(lg) = float2{v[0], v[1]};
+        else *lg = v[0];
+      }
     }
   __syncthreads();
   // selection: token tid / L, lane part tid % L scans experts part, part + L, ... (ascending) into a sorted list of
-  // its best KL = 8 (k <= 8, so a lane's share of the top k is always in it; the rest never matter)
-  constexpr int KL = 8;
+  // its best KL = 8 (k <= 8, so a lane's share of the top k is always in it; the rest never matter), or all of them
+  constexpr int KL = EPL < 8 ? EPL : 8;
   const int tt = tid / L, part = tid % L, t = t0 + tt;
   float tv[KL];
   int ti[KL];
@@ -644,24 +655,31 @@ int lsurge::router_topk_impl(const void* x, const void* w_r, const float* bias, 
     // E = 256, d = 2048 700 / 629 / 613
     const int64_t chunks = (t + 63) / 64, per16 = chunks * 4 * (e / 32);  // waves at one tile each
     const int tt = per16 / 4 >= 2048 ? 4 : per16 / 2 >= 2048 ? 2 : 1;
+    // one expert tile a wave while its waves (E / 16 a workgroup) have a SIMD each: the logits' chain is then half as
+    // many matrix steps.  Alone, cold: T = 64 / 1024 / 4096, E = 64 20.5 / 19.8 / 20.4 -> 15.6 / 15.0 / 16.1 us; T = 64,
+    // E = 32 18.5 -> 13.9.  With more waves than SIMDs the steps only move between waves (T = 16384, E = 64 34 -> 37
+    // us; E = 128, whose eight waves share a CU's four SIMDs, 20.6 -> 20.5)
+    const bool narrow = e <= 64 && chunks * 4 * (e / 16) <= 1024;
     const dim3 grid((unsigned)(chunks * (4 / tt)));  // whole chunks: every byte of hist is written
-#define RF_LAUNCH(E_, TT_, DC_)                                                                                    \
+#define RF_LAUNCH(E_, TT_, HT_, DC_)                                                                                   \
   LSURGE_LAUNCH(KID_ROUTER, s,                                                                                     \
-                hipLaunchKernelGGL((router_fused_kernel<E_, TT_, DC_>), grid, dim3(2 * E_), 0, s, (const bf16_t*)x, \
+                hipLaunchKernelGGL((router_fused_kernel<E_, TT_, HT_, DC_>), grid, dim3(4 * E_ / HT_), 0, s, (const bf16_t*)x, \
                                    (const bf16_t*)w_r, bias, (int)t, (int)d, (int)k, logits, sel, weights,         \
                                    (uint8_t*)hist))
-#define RF_DC(E_, TT_)                          \
-  do {                                          \
-    if (d % 128 == 0) RF_LAUNCH(E_, TT_, 128);  \
-    else RF_LAUNCH(E_, TT_, 64);                \
+#define RF_DC(E_, TT_, HT_)                          \
+  do {                                               \
+    if (d % 128 == 0) RF_LAUNCH(E_, TT_, HT_, 128);  \
+    else RF_LAUNCH(E_, TT_, HT_, 64);                \
   } while (0)
-#define RF_CASE(E_)                 \
-  do {                              \
-    if (tt == 4) RF_DC(E_, 4);      \
-    else if (tt == 2) RF_DC(E_, 2); \
-    else RF_DC(E_, 1);              \
+#define RF_CASE(E_)                    \
+  do {                                 \
+    if (tt == 4) RF_DC(E_, 4, 2);      \
+    else if (tt == 2) RF_DC(E_, 2, 2); \
+    else RF_DC(E_, 1, 2);              \
   } while (0)
-    if (e == 32) RF_CASE(32);
+    if (narrow && e == 32) RF_DC(32, 1, 1);
+    else if (narrow) RF_DC(64, 1, 1);
+    else if (e == 32) RF_CASE(32);
     else if (e == 64) RF_CASE(64);
     else if (e == 128) RF_CASE(128);
     else RF_CASE(256);

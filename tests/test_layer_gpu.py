@@ -149,6 +149,14 @@ def test_fused_router_matrix_core_chain(T, d, E, k, dev):
         assert np.array_equal(v[n], lay[n]), n
 
 
+@pytest.mark.parametrize("T,d,E,k", [(4096, 64, 64, 2), (4097, 64, 64, 2), (8192, 128, 32, 1), (8193, 64, 32, 3),
+                                     (448, 64, 32, 8), (449, 64, 64, 2), (512, 192, 32, 2), (513, 64, 128, 3)])
+def test_fused_router_narrow_tiles_and_layout_workgroups(T, d, E, k, dev):
+    """Both sides of the router's one-expert-tile rule (a wave per SIMD: T = 4096 at 64 experts, 8192 at 32), and of the
+    layout's least number of workgroups (7 and 8 chunks of 64 tokens): the split router's bits, the oracle's layout."""
+    test_fused_router_matrix_core_chain(T, d, E, k, dev)
+
+
 def test_hot_experts_chunked_wgrad(dev):
     """Every token routes to experts 0 and 1 (a large bias), so each holds 5000 rows: the routed weight gradients
     cut them into 4096 + 904-row chunks summed from partials, and the six empty experts get zero gradients."""
