@@ -72,6 +72,36 @@ __device__ __forceinline__ int block_scan_excl(int v, int* ws, int* total) {
   return base + x - v;
 }
 
+// Three of them at once, through 48 entries of LDS scratch and one barrier (none at the end: the caller has one before
+// ws is used again).
+__device__ __forceinline__ void block_scan3_excl(int v0, int v1, int v2, int* ws, int (&pre)[3], int (&tot)[3]) {
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, nw = (int)blockDim.x >> 6;
+  const int v[3] = {v0, v1, v2};
+  int x[3] = {v0, v1, v2};
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1)
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const int y = __shfl_up(x[q], o, 64);
+      if (lane >= o) x[q] += y;
+    }
+  if (lane == 63)
+#pragma unroll
+    for (int q = 0; q < 3; ++q) ws[16 * q + w] = x[q];
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    int base = 0, all = 0;
+    for (int i = 0; i < nw; ++i) {
+      const int t = ws[16 * q + i];
+      if (i < w) base += t;
+      all += t;
+    }
+    tot[q] = all;
+    pre[q] = base + x[q] - v[q];
+  }
+}
+
 // The scan's tables from the expert-level results in LDS (gs_s [E], boff_s and tb_s [E + 1]: block and 256-row tile
 // bases, totals last): the block table, the padding markers of row_src, the tile table and the shared expert's
 // row_src, each over its entries i0, i0 + stride, ... (one workgroup's threads, or those of every workgroup).
@@ -343,28 +373,36 @@ __global__ __launch_bounds__(1024) void layout_rank_kernel(
 // The whole layout in one launch, for the layer when the fused router made the chunk histograms and they are small
 // (nchunk E <= LF_HIST_MAX): every workgroup sums the histograms itself (the chunks before its own give its
 // per-expert rank bases, all of them the expert totals), so no scan kernel runs between the router and the ranks.
-// The scan's tables are spread over all workgroups, and the last one writes the weight gradients' chunk table.
+// Workgroup c < nchunk ranks chunk c, one slot a thread.  The scan's tables are spread over all workgroups, of which
+// there are at least LF_MIN_WG, and the last one, which has no slots, writes the weight gradients' chunk table.
 // Needs E + 1 <= blockDim.x: a thread per expert in the expert-level scans, and one more for the chunk table's
 // extra expert.  Each workgroup reads nchunk E ints of histograms (64 KB at T = 16384 tokens, 64 experts), from L2.
-constexpr int LF_HIST_MAX = 32768, LF_LOADS = 16;
+//
+// Bound by its chain of barriers and first loads, so the slots are loaded and counted (per wave: the 64 lanes' peers
+// by ballots, the highest one writing the count, no atomics) beside the histogram loads, one scan carries the three
+// expert-level sums, and the chunk table's three scans are off the ranking workgroups.
+// Measured (kernel trace of the layer's forward, 64 experts, k = 6): T = 64 13.4 -> 7.8 us, T = 4096 13.4 -> 10.7; at
+// T = 16384, where it runs beside the shared expert's GEMM, 24 us as before.
+constexpr int LF_HIST_MAX = 32768, LF_LOADS = 16, LF_MIN_WG = 8;
 __global__ __launch_bounds__(1024) void layout_fused_kernel(
     const int32_t* __restrict__ flat, int64_t M, int E, const int32_t* __restrict__ hist, int nchunk, int nbits,
-    int per_wave, int32_t* __restrict__ order, int32_t* __restrict__ pos, int32_t* __restrict__ slot,
+    int32_t* __restrict__ order, int32_t* __restrict__ pos, int32_t* __restrict__ slot,
     int32_t* __restrict__ row_src, int32_t* __restrict__ group_sizes, int32_t* __restrict__ offsets,
     int32_t* __restrict__ block_off, int32_t* __restrict__ blk_expert, int32_t* __restrict__ blk_rows,
     int32_t* __restrict__ num_blocks, int max_blocks, lsurge::LayoutTiles tiles) {
   extern __shared__ int32_t sh[];
-  const int tid = threadIdx.x, nt = (int)blockDim.x, nw = nt >> 6, me = (int)blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nt = (int)blockDim.x, nw = nt >> 6, me = (int)blockIdx.x;
   const int tpe = nt / E;               // threads per expert in the histogram sums
   int32_t* cnt = sh;                    // [nw][E]
   int32_t* part = cnt + nw * E;         // [2][tpe][E]: partial sums below this chunk, and over all chunks
-  int32_t* below_s = part + 2 * tpe * E;
-  int32_t* gs_s = below_s + E;
+  int32_t* gs_s = part + 2 * tpe * E;
   int32_t* off_s = gs_s + E;
   int32_t* boff_s = off_s + E;          // [E + 1]
   int32_t* tb_s = boff_s + E + 1;       // [E + 1]
-  int32_t* ws = tb_s + E + 1;           // [16]
-  for (int i = tid; i < nw * E; i += nt) cnt[i] = 0;
+  int32_t* ws = tb_s + E + 1;           // [48]
+  const int64_t i = (int64_t)me * nt + tid;  // this thread's slot
+  const int fe = me < nchunk && i < M ? flat[i] : -1;
+  for (int e = lane; e < E; e += 64) cnt[wv * E + e] = 0;  // this wave's row: in order with the counts below
   const int e_t = tid % E, j_t = tid / E;
   if (j_t < tpe) {
     int below = 0, all = 0;
@@ -385,41 +423,53 @@ __global__ __launch_bounds__(1024) void layout_fused_kernel(
     part[j_t * E + e_t] = below;
     part[(tpe + j_t) * E + e_t] = all;
   }
+  const bool valid = fe >= 0 && fe < E;  // ids outside [0, E) are skipped, as in rank_chunk
+  uint64_t peers = peers_of(valid ? fe : (1 << nbits) - 1, nbits) & __ballot(valid);
+  if (!valid) peers = 0;
+  const int rank_in = __popcll(peers & ((lane == 0) ? 0ull : (~0ull >> (64 - lane))));
+  __builtin_amdgcn_wave_barrier();
+  if (valid && (peers >> lane) == 1ull) cnt[wv * E + fe] = rank_in + 1;
   __syncthreads();
-  if (tid < E) {
-    int below = 0, all = 0;
+  int below = 0, g = 0;
+  if (tid < E)
     for (int j = 0; j < tpe; ++j) {
       below += part[j * E + tid];
-      all += part[(tpe + j) * E + tid];
+      g += part[(tpe + j) * E + tid];
     }
-    below_s[tid] = below;
-    gs_s[tid] = all;
-  }
-  __syncthreads();
-  // expert offsets, block offsets and tile bases: the same scans as the scan kernel's
-  const int g = tid < E ? gs_s[tid] : 0;
-  int tot, nbt, ntt = 0;
-  const int off = block_scan_excl(g, ws, &tot);
-  const int boff = block_scan_excl((g + BLK - 1) / BLK, ws, &nbt);
-  const int tbase = tiles.t_expert ? block_scan_excl((g + 2 * BLK - 1) / (2 * BLK), ws, &ntt) : 0;
+  // expert offsets, block offsets and tile bases: the scan kernel's sums, in one scan
+  int pre[3], tot[3];
+  block_scan3_excl(g, (g + BLK - 1) / BLK, (g + 2 * BLK - 1) / (2 * BLK), ws, pre, tot);
   if (tid < E) {
-    off_s[tid] = off;
-    boff_s[tid] = boff;
-    tb_s[tid] = tbase;
+    gs_s[tid] = g;
+    off_s[tid] = pre[0];
+    boff_s[tid] = pre[1];
+    tb_s[tid] = pre[2];
     if (me == 0) {
       if (group_sizes) group_sizes[tid] = g;
-      if (offsets) offsets[tid] = off;
-      if (block_off) block_off[tid] = boff;
+      if (offsets) offsets[tid] = pre[0];
+      if (block_off) block_off[tid] = pre[1];
+    }
+    for (int w = 0; w < nw; ++w) {  // the waves' first ranks
+      const int v = cnt[w * E + tid];
+      cnt[w * E + tid] = below;
+      below += v;
     }
   }
   if (tid == 0) {
-    boff_s[E] = nbt;
-    tb_s[E] = ntt;
+    boff_s[E] = tot[1];
+    tb_s[E] = tot[2];
   }
   __syncthreads();
-  rank_chunk(
-      flat, M, E, cnt, [&](int e) { return below_s[e]; }, [&](int e) { return off_s[e]; },
-      [&](int e) { return boff_s[e]; }, nbits, per_wave, order, pos, slot, row_src);
+  if (valid) {
+    const int rank = cnt[wv * E + fe] + rank_in, p = off_s[fe] + rank;
+    if (pos) pos[i] = p;
+    if (order) order[p] = (int32_t)i;
+    if (slot) {
+      const int sl = BLK * boff_s[fe] + rank;
+      slot[i] = sl;
+      if (row_src) row_src[sl] = (int32_t)i;
+    }
+  }
   write_layout_tables(E, gs_s, boff_s, tb_s, row_src, blk_expert, blk_rows, num_blocks, max_blocks, tiles,
                       me * nt + tid, (int)gridDim.x * nt);
   if (tiles.chunks.c_expert && me == (int)gridDim.x - 1)
@@ -476,11 +526,12 @@ int layout_common(const int32_t* flat, int64_t M, int64_t E, int32_t* gs, int32_
   // the fused router's histograms, when small: the whole layout in one launch (layout_fused_kernel)
   if (pre.hist && 64 * waves >= E + 1 && nchunk * E <= LF_HIST_MAX) {
     const int nt = 64 * waves, tpe = nt / (int)E;
-    const size_t lds = sizeof(int32_t) * ((size_t)waves * E + 2 * (size_t)tpe * E + 5 * (size_t)E + 2 + 16);
+    const size_t lds = sizeof(int32_t) * ((size_t)waves * E + 2 * (size_t)tpe * E + 4 * (size_t)E + 2 + 48);
+    const unsigned wgs = (unsigned)std::max<int64_t>(nchunk + 1, LF_MIN_WG);
     LSURGE_LAUNCH(KID_LAYOUT_RANK, s,
-                  hipLaunchKernelGGL(layout_fused_kernel, dim3((unsigned)nchunk), dim3(nt), lds, s, flat, M, (int)E,
-                                     hist, (int)nchunk, nbits, per_wave, order, pos, slot, row_src, gs, offsets,
-                                     block_off, blk_expert, blk_rows, num_blocks, (int)max_blocks, tiles));
+                  hipLaunchKernelGGL(layout_fused_kernel, dim3(wgs), dim3(nt), lds, s, flat, M, (int)E, hist,
+                                     (int)nchunk, nbits, order, pos, slot, row_src, gs, offsets, block_off,
+                                     blk_expert, blk_rows, num_blocks, (int)max_blocks, tiles));
     return LSURGE_OK;
   }
   if (!pre.hist)
