@@ -1,4 +1,4 @@
-// Router: f32 logits (sequential sum over d), top-k with lower-index tie-break, softmax over the selection.
+// Router: f32 logits (sequential sum over d), top-k with lower-index tie-break (topk.h), softmax over the selection.
 //
 // Stands in for MaxText RoutedMoE's gate + top-k (third-party; configured by configs/stage1.yml:34-37 of the
 // reference).  Logit order contract: logits[t,e] = (((x[t,0]w[0,e]) + x[t,1]w[1,e]) + ...) in f32, then
@@ -11,9 +11,44 @@
 // of 16 to 64 tokens x all experts computing the same logits on the f32 matrix cores, then top-k, softmax and the
 // layout's per-64-token expert histograms in the same workgroup (described at the kernel).
 #include "launchers.h"
-
+#include "topk.h"
 
 namespace {
+
+using lsurge::TOPK_NO_ID;
+using lsurge::TOPK_NO_KEY;
+using lsurge::TopkList;
+using lsurge::topk_before;
+using lsurge::topk_key;
+using lsurge::topk_logit;
+
+// One round of a wave-per-token selection over the wave's keys (lane + 64 c is expert lane + 64 c of the token): the
+// best candidate, the same in every lane, whose key is then removed.
+template <int EC>
+__device__ __forceinline__ void wave_take_best(uint32_t (&key)[EC], int lane, uint32_t* bk_out, int* bi_out) {
+  uint32_t bk = TOPK_NO_KEY;
+  int bi = TOPK_NO_ID;
+#pragma unroll
+  for (int c = 0; c < EC; ++c)
+    if (key[c] > bk) {  // ascending experts: strictly larger keeps the lower index of a tie
+      bk = key[c];
+      bi = lane + 64 * c;
+    }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint32_t ok = __shfl_xor(bk, o, 64);
+    const int oi = __shfl_xor(bi, o, 64);
+    if (topk_before(ok, oi, bk, bi)) {
+      bk = ok;
+      bi = oi;
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < EC; ++c)
+    if (lane + 64 * c == bi) key[c] = TOPK_NO_KEY;
+  *bk_out = bk;
+  *bi_out = bi;
+}
 
 constexpr int RT_TOK = 64;       // tokens per workgroup
 constexpr int RT_DC = 32;        // d chunk staged in LDS
@@ -105,40 +140,18 @@ __global__ __launch_bounds__(RT_THREADS) void router_topk_kernel(const bf16_t* _
     const int t = t0 + tt;
     if (t >= T) break;
     constexpr int EC = (EP + 63) / 64;
-    float v[EC];
-    bool taken[EC];
+    uint32_t key[EC];
 #pragma unroll
     for (int c = 0; c < EC; ++c) {
       const int e = lane + 64 * c;
-      v[c] = (e < E) ? ls[tt * EP + e] : -INFINITY;
-      taken[c] = !(e < E);
+      key[c] = (e < E) ? topk_key(ls[tt * EP + e]) : TOPK_NO_KEY;
     }
     float top0 = 0.f, denom = 0.f;
     for (int j = 0; j < k; ++j) {
-      // lane-local best (lowest index wins ties: c ascending, strict >)
-      float bv = -INFINITY;
-      int bi = 0x7fffffff;
-#pragma unroll
-      for (int c = 0; c < EC; ++c) {
-        const int e = lane + 64 * c;
-        if (!taken[c] && (bi == 0x7fffffff || v[c] > bv)) {
-          bv = v[c];
-          bi = e;
-        }
-      }
-      // wave argmax: larger value, then lower index
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(bv, o, 64);
-        const int oi = __shfl_xor(bi, o, 64);
-        if (oi != 0x7fffffff && (bi == 0x7fffffff || ov > bv || (ov == bv && oi < bi))) {
-          bv = ov;
-          bi = oi;
-        }
-      }
-#pragma unroll
-      for (int c = 0; c < EC; ++c)
-        if (lane + 64 * c == bi) taken[c] = true;
+      uint32_t bk;
+      int bi;
+      wave_take_best(key, lane, &bk, &bi);
+      const float bv = topk_logit(bk);
       if (j == 0) top0 = bv;
       const float z = __expf(bv - top0);
       denom += z;
@@ -309,9 +322,8 @@ __global__ __launch_bounds__(RL_THREADS) void router_logits_kernel(const bf16_t*
 // Then, in the same workgroup:
 //  - the logits go to HBM and to an LDS tile [TOK][E + 1];
 //  - top-k + softmax per token: L = E / (4 HT TT) lanes per token each keep a sorted list of the best 8 of their
-//    EPL = 4 HT TT experts (scanned in ascending expert order, a logit moves ahead only of strictly smaller ones), and
-//    k merge rounds take the best head of the L lists (larger logit, ties to the lower expert index) -- the order of
-//    a stable descending sort, as in router_select_lane_kernel, whose softmax (in rank order) this repeats;
+//    EPL = 4 HT TT experts (scanned in ascending expert order), and k merge rounds take the best head of the L lists, in
+//    the order of topk.h, as router_select_lane_kernel, whose softmax (in rank order) this repeats;
 //  - the expert histogram of the workgroup's TOK k slots (LDS counters) -> hist[chunk of 64 tokens][E], the layout's
 //    per-chunk counts.  A word of hist holds the counts of its chunk's four 16-token quarters in its bytes (a token
 //    picks an expert at most once, so even 64 tokens fit one byte): a workgroup writes the TT bytes of its own
@@ -436,57 +448,36 @@ __global__ __launch_bounds__(4 * E / HT, E == 256 ? 4 : 1) void router_fused_ker
   // selection: token tid / L, lane part tid % L scans experts part, part + L, ... (ascending) into a sorted list of
   // its best KL = 8 (k <= 8, so a lane's share of the top k is always in it; the rest never matter), or all of them
   constexpr int KL = EPL < 8 ? EPL : 8;
+  static_assert(L * KL >= 8, "the lists of a token hold its k <= 8 experts");
   const int tt = tid / L, part = tid % L, t = t0 + tt;
-  float tv[KL];
-  int ti[KL];
-#pragma unroll
-  for (int j = 0; j < KL; ++j) {
-    tv[j] = 0.f;
-    ti[j] = -1;
-  }
+  TopkList<KL> list;
+  list.clear();
 #pragma unroll 1
   for (int c = 0; c < EPL; ++c) {
     const int e = part + L * c;
-    float cv = lt[tt * (E + 1) + e];
-    int ci = e;
-    bool placed = false;
-#pragma unroll
-    for (int j = 0; j < KL; ++j) {
-      const bool g = placed || ti[j] < 0 || cv > tv[j];
-      const float ov = tv[j];
-      const int oi = ti[j];
-      tv[j] = g ? cv : ov;
-      ti[j] = g ? ci : oi;
-      cv = g ? ov : cv;
-      ci = g ? oi : ci;
-      placed = g;
-    }
+    list.insert(topk_key(lt[tt * (E + 1) + e]), e);
   }
-  // k merge rounds over the L lanes of the token (an aligned group of L lanes of one wave)
+  // k merge rounds over the L lanes of the token (an aligned group of L lanes of one wave).  The order is total, so the
+  // lanes agree on the winner whatever the logits are, and exactly one of them advances: k distinct experts of [0, E)
   float top0 = 0.f, denom = 0.f, zj[8];
   int sj[8];
   int head = 0;
   for (int j = 0; j < k; ++j) {
-    float hv = 0.f;
-    int hi = -1;
-#pragma unroll
-    for (int q = 0; q < KL; ++q)
-      if (q == head) {
-        hv = tv[q];
-        hi = ti[q];
-      }
-    float bv = hv;
+    uint32_t bk;
+    int hi;
+    list.get(head, &bk, &hi);
     int bi = hi;
 #pragma unroll
     for (int o = 1; o < L; o <<= 1) {
-      const float ov = __shfl_xor(bv, o, 64);
+      const uint32_t ok = __shfl_xor(bk, o, 64);
       const int oi = __shfl_xor(bi, o, 64);
-      if (oi >= 0 && (bi < 0 || ov > bv || (ov == bv && oi < bi))) {
-        bv = ov;
+      if (topk_before(ok, oi, bk, bi)) {
+        bk = ok;
         bi = oi;
       }
     }
-    if (hi == bi && hi >= 0) ++head;  // the lane that held the winner advances
+    if (hi == bi) ++head;  // the lane that held the winner advances
+    const float bv = topk_logit(bk);
     if (j == 0) top0 = bv;
     const float z = __expf(bv - top0);
     denom += z;
@@ -518,45 +509,25 @@ __global__ __launch_bounds__(4 * E / HT, E == 256 ? 4 : 1) void router_fused_ker
   }
 }
 
-// one wave per token: top-k (larger logit first, ties to the lower expert index), softmax over the k
+// one wave per token: top-k (the order of topk.h), softmax over the k
 template <int EC>  // logits per lane: E <= 64 EC
 __global__ __launch_bounds__(256) void router_select_kernel(const float* __restrict__ logits, int T, int E, int k,
                                                             int32_t* __restrict__ sel, float* __restrict__ weights) {
   const int lane = threadIdx.x & 63;
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= T) return;
-  float v[EC];
-  bool taken[EC];
+  uint32_t key[EC];
 #pragma unroll
   for (int c = 0; c < EC; ++c) {
     const int e = lane + 64 * c;
-    v[c] = (e < E) ? logits[(int64_t)t * E + e] : -INFINITY;
-    taken[c] = !(e < E);
+    key[c] = (e < E) ? topk_key(logits[(int64_t)t * E + e]) : TOPK_NO_KEY;
   }
   float top0 = 0.f, denom = 0.f, mine = 0.f;
   for (int j = 0; j < k; ++j) {
-    float bv = -INFINITY;
-    int bi = 0x7fffffff;
-#pragma unroll
-    for (int c = 0; c < EC; ++c) {
-      const int e = lane + 64 * c;
-      if (!taken[c] && (bi == 0x7fffffff || v[c] > bv)) {
-        bv = v[c];
-        bi = e;
-      }
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ov = __shfl_xor(bv, o, 64);
-      const int oi = __shfl_xor(bi, o, 64);
-      if (oi != 0x7fffffff && (bi == 0x7fffffff || ov > bv || (ov == bv && oi < bi))) {
-        bv = ov;
-        bi = oi;
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < EC; ++c)
-      if (lane + 64 * c == bi) taken[c] = true;
+    uint32_t bk;
+    int bi;
+    wave_take_best(key, lane, &bk, &bi);
+    const float bv = topk_logit(bk);
     if (j == 0) top0 = bv;
     const float z = __expf(bv - top0);
     denom += z;
@@ -566,10 +537,9 @@ __global__ __launch_bounds__(256) void router_select_kernel(const float* __restr
   if (lane < k) weights[(int64_t)t * k + lane] = mine / denom;
 }
 
-// one lane per token: the k largest logits (ties -> lower expert index) kept in a sorted register list while the
-// token's logits are scanned in ascending expert order, then the softmax over them in rank order.  A new logit
-// enters at the first slot whose logit it strictly exceeds (or the first empty slot); everything below shifts down,
-// so equal logits stay in ascending expert order.  K >= k is the list's compile-time size.
+// one lane per token: the k best logits (the order of topk.h) kept in a sorted register list while the token's logits
+// are scanned in ascending expert order, then the softmax over them in rank order.  K >= k is the list's compile-time
+// size.
 template <int K>
 __global__ __launch_bounds__(256) void router_select_lane_kernel(const float* __restrict__ logits, int T, int E, int k,
                                                                  int32_t* __restrict__ sel,
@@ -577,29 +547,9 @@ __global__ __launch_bounds__(256) void router_select_lane_kernel(const float* __
   const int t = blockIdx.x * 256 + threadIdx.x;
   if (t >= T) return;
   const float* l = logits + (int64_t)t * E;
-  float tv[K];
-  int ti[K];
-#pragma unroll
-  for (int j = 0; j < K; ++j) {
-    tv[j] = 0.f;
-    ti[j] = -1;
-  }
-  auto insert = [&](float v, int e) {
-    bool placed = false;
-    float cv = v;
-    int ci = e;
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-      const bool g = placed || ti[j] < 0 || cv > tv[j];
-      const float ov = tv[j];
-      const int oi = ti[j];
-      tv[j] = g ? cv : ov;
-      ti[j] = g ? ci : oi;
-      cv = g ? ov : cv;
-      ci = g ? oi : ci;
-      placed = g;
-    }
-  };
+  TopkList<K> best;
+  best.clear();
+  auto insert = [&](float v, int e) { best.insert(topk_key(v), e); };
   if ((E & 3) == 0) {
     for (int e = 0; e < E; e += 4) {
       const f32x4 q = *reinterpret_cast<const f32x4*>(l + e);
@@ -613,14 +563,15 @@ __global__ __launch_bounds__(256) void router_select_lane_kernel(const float* __
   }
   // softmax over the k best, denominator summed in rank order
   float denom = 0.f;
+  const float top0 = topk_logit(best.key[0]);
 #pragma unroll
   for (int j = 0; j < K; ++j)
-    if (j < k) denom += __expf(tv[j] - tv[0]);
+    if (j < k) denom += __expf(topk_logit(best.key[j]) - top0);
 #pragma unroll
   for (int j = 0; j < K; ++j) {
     if (j < k) {
-      sel[(int64_t)t * k + j] = ti[j];
-      weights[(int64_t)t * k + j] = __expf(tv[j] - tv[0]) / denom;
+      sel[(int64_t)t * k + j] = best.id[j];
+      weights[(int64_t)t * k + j] = __expf(topk_logit(best.key[j]) - top0) / denom;
     }
   }
 }

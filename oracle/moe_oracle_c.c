@@ -7,7 +7,7 @@
  *  oracle_router_logits  logits[t,e] = sum_i x[t,i] * w[i,e], summed sequentially over i in float32,
  *                        then + bias[e] (MaxText RoutedMoE gate; numerics contract of moe_oracle.py).
  *  oracle_topk           k largest logits per token, descending, ties -> lower expert index
- *                        (argsort(-logits)[:, :k] as in modal/test_moe_permute.py:23-26).
+ *                        (argsort(-logits)[:, :k] as in modal/test_moe_permute.py:23-26), NaN last.
  *  oracle_layout         stable counting sort of the flat slots by expert (modal/moe_permute.py:240-264)
  *                        plus the 128-row padded block layout.
  */
@@ -52,7 +52,8 @@ void oracle_topk(const float* logits, int64_t T, int64_t E, int64_t k, int32_t* 
       int64_t best = -1;
       for (int64_t e = 0; e < E; ++e) {
         if (taken[e]) continue;
-        if (best < 0 || l[e] > l[best]) best = e; /* strict '>' keeps the lower index on ties */
+        /* strict '>' keeps the lower index on ties; NaN sorts last, as in numpy's argsort */
+        if (best < 0 || l[e] > l[best] || (l[best] != l[best] && l[e] == l[e])) best = e;
       }
       taken[best] = 1;
       sel[t * k + j] = (int32_t)best;

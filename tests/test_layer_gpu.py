@@ -157,6 +157,60 @@ def test_fused_router_narrow_tiles_and_layout_workgroups(T, d, E, k, dev):
     test_fused_router_matrix_core_chain(T, d, E, k, dev)
 
 
+@pytest.mark.parametrize("T,E,k", [(64, 64, 8), (4096, 64, 6), (4097, 64, 6), (8192, 32, 8), (8193, 32, 8), (300, 128, 8),
+                                   (300, 256, 8), (300, 16, 4), (8200, 16, 4), (70, 40, 12)])
+def test_nan_tokens_and_experts(T, E, k, dev):
+    """NaN logits: every logit of some tokens (a NaN in their row of x) and those of three experts on all tokens (NaN
+    columns of W_r).  Each token still gets k distinct experts of [0, E), the numbers in order and then the NaN by
+    index, on both sides of the fused router's one-expert-tile rule and on the split selections; the NaN tokens' outputs
+    and input gradients are NaN, and every other token's have the bits of the same call without NaN tokens."""
+    from test_router_layout_gpu import gpu_router
+    d, f = 128, 64
+    p = mo.make_inputs(T=T, d=d, E=E, k=k, f=f, fs=64, seed=E + k)
+    p["w_r"][3, [1, E // 2, E - 1]] = np.nan
+    nan = np.zeros(T, bool)
+    nan[[0, 1, T // 2, T - 1]] = True
+    res = []
+    for bad in (False, True):
+        x = p["x"].copy()
+        x[nan, 7] = np.nan if bad else 0.0
+        q = dict(p, x=x)
+        tp = to_dev(q, dev)
+        layer = MoELayer(MoEShape(T, d, E, k, f, 64), dev)
+        layer.saved.fill_(0xFF)  # ids and slots that are not written are out of range
+        out = layer.forward(tp).clone()
+        v = {n: t.cpu().numpy() for n, t in layer.views().items() if t.dtype != torch.bfloat16}
+        assert v["sel"].min() >= 0 and v["sel"].max() < E
+        assert np.array_equal(v["sel"], mo.topk_lower_index(v["logits"], k))
+        logits_s, sel_s, wts_s = gpu_router(x, p["w_r"], k, p["bias"], dev)
+        assert np.array_equal(np.isnan(v["logits"]), np.isnan(logits_s))
+        assert np.array_equal(v["sel"], sel_s)
+        assert np.array_equal(v["weights"], wts_s, equal_nan=True)
+        lay = co.build_layout(v["sel"], E)
+        for n in ("group_sizes", "offsets", "block_off", "order", "pos", "slot"):
+            assert np.array_equal(v[n], lay[n]), n
+        dy = torch.from_numpy(p["dy"]).to(dev).to(torch.bfloat16)
+        res.append((out, layer.backward(tp, dy)["dx"].clone()))
+    keep = torch.from_numpy(~nan).to(dev)
+    for clean, got in zip(*res):
+        assert torch.isfinite(clean).all()
+        assert torch.equal(got[keep], clean[keep])
+        assert torch.isnan(got[~keep]).all()
+
+
+@pytest.mark.parametrize("T,E,k", [(70, 256, 80), (70, 100, 65)])
+def test_nan_logits_one_kernel_router(T, E, k, dev):
+    """The router in one kernel (k > 64) on NaN logits: the stable descending order, NaN last."""
+    from test_router_layout_gpu import gpu_router
+    rng = np.random.default_rng(E)
+    x, w_r = rng.standard_normal((T, 32)).astype(np.float32), rng.standard_normal((32, E)).astype(np.float32)
+    x, w_r = mo.round_bf16(x), mo.round_bf16(w_r)
+    x[3, 4] = np.nan
+    w_r[5, ::3] = np.nan
+    logits, sel, _ = gpu_router(x, w_r, k, None, dev)
+    assert np.array_equal(sel, mo.topk_lower_index(logits, k))
+
+
 def test_hot_experts_chunked_wgrad(dev):
     """Every token routes to experts 0 and 1 (a large bias), so each holds 5000 rows: the routed weight gradients
     cut them into 4096 + 904-row chunks summed from partials, and the six empty experts get zero gradients."""
