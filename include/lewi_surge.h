@@ -331,7 +331,8 @@ int lsurge_moe_fwd_fp8(const lsurge_moe_shape* s, const lsurge_moe_params* p, co
  * and [dG | dU] over all routed rows, the shared expert's dY and [dG | dU] on their own.  dgrads: E5M2 x the
  * weights' E4M3 codes (each weight at its own scale); wgrads: the forward's E4M3 codes of h and x (same
  * scales) x the E5M2 gradients.  Combine, dispatch and router backward are those of lsurge_moe_bwd; the
- * gradients come out in the same buffers and dtypes.  p needs x and w_r (the bf16 expert weights are not
+ * gradients come out in the same buffers and dtypes, the weight gradients in f32 (not lsurge_moe_bwd_as's bf16: its
+ * buffers hold half of what is written here).  p needs x and w_r (the bf16 expert weights are not
  * read). */
 size_t lsurge_moe_bwd_fp8_workspace_bytes(const lsurge_moe_shape* s);
 int lsurge_moe_bwd_fp8(const lsurge_moe_shape* s, const lsurge_moe_params* p, const void* wq, size_t wq_bytes,

@@ -14,6 +14,7 @@ router w_r [d, E]; shared expert ws_gate/ws_up [d, fs], ws_down [fs, d].
 from __future__ import annotations
 
 import ctypes
+import math
 from dataclasses import dataclass
 
 import torch
@@ -59,6 +60,33 @@ def _check_params(s: MoEShape, p: dict):
     b = p.get("bias")
     if b is not None and (tuple(b.shape) != (s.e,) or b.dtype != torch.float32 or not b.is_cuda):
         raise ValueError("moe_layer: bias must be a float32 ROCm tensor of shape (e,)")
+
+
+def _grad_shapes(s: MoEShape):
+    g = dict(dx=(s.t, s.d), dw_r=(s.d, s.e), dw_gate=(s.e, s.d, s.f), dw_up=(s.e, s.d, s.f), dw_down=(s.e, s.f, s.d),
+             dweights=(s.t, s.k))
+    if s.fs:
+        g.update(dws_gate=(s.d, s.fs), dws_up=(s.d, s.fs), dws_down=(s.fs, s.d))
+    return g
+
+
+def _check_grads(s: MoEShape, grads: dict, dw_dtypes):
+    """The dtype of the weight-gradient buffers, one of dw_dtypes; every buffer must hold what the kernels write."""
+    dw = None
+    for n, shp in _grad_shapes(s).items():
+        t = grads.get(n)
+        if t is None:  # the C call says which ones it needs
+            continue
+        if n.startswith("dw") and n != "dweights":
+            if dw is not None and t.dtype != dw:
+                raise ValueError("moe_layer: the weight gradients must share one dtype")
+            dw, want = t.dtype, dw_dtypes
+        else:
+            want = (torch.bfloat16,) if n == "dx" else (torch.float32,)
+        if t.dtype not in want or not t.is_contiguous() or t.numel() < math.prod(shp):
+            raise ValueError(f"moe_layer: {n} must be a contiguous buffer of {math.prod(shp)} values of "
+                             f"{' or '.join(str(d) for d in want)}, got {tuple(t.shape)} {t.dtype}")
+    return dw or torch.float32
 
 
 def _params_struct(p: dict):
@@ -133,15 +161,11 @@ class MoELayer:
         return out
 
     def alloc_grads(self, dw_dtype=torch.float32):
-        """Gradient buffers for backward(): dx bf16, dweights f32, the weight gradients in dw_dtype (f32 or bf16)."""
-        s = self.shape
-        z = lambda *shape: torch.empty(shape, dtype=dw_dtype, device=self.device)  # noqa: E731
-        g = dict(dx=torch.empty((s.t, s.d), dtype=torch.bfloat16, device=self.device), dw_r=z(s.d, s.e),
-                 dw_gate=z(s.e, s.d, s.f), dw_up=z(s.e, s.d, s.f), dw_down=z(s.e, s.f, s.d),
-                 dweights=torch.empty((s.t, s.k), dtype=torch.float32, device=self.device))
-        if s.fs:
-            g.update(dws_gate=z(s.d, s.fs), dws_up=z(s.d, s.fs), dws_down=z(s.fs, s.d))
-        return g
+        """Gradient buffers for backward(): dx bf16, dweights f32, the weight gradients in dw_dtype (f32, or bf16, which
+        backward_fp8() does not write)."""
+        other = dict(dx=torch.bfloat16, dweights=torch.float32)
+        return {n: torch.empty(shp, dtype=other.get(n, dw_dtype), device=self.device)
+                for n, shp in _grad_shapes(self.shape).items()}
 
     def backward(self, p: dict, dy, grads=None):
         """Gradients into `grads` (alloc_grads(); by default this layer's own f32 ones): weight gradients in their
@@ -154,21 +178,19 @@ class MoELayer:
             if self.grads is None:
                 self.grads = self.alloc_grads()
             grads = self.grads
-        dw = [grads[n] for n in GRAD_NAMES if n.startswith("dw") and n != "dweights" and grads.get(n) is not None]
-        if len({t.dtype for t in dw}) > 1:
-            raise ValueError("moe_layer: the weight gradients must share one dtype")
+        dw = _check_grads(s, grads, (torch.float32, torch.bfloat16))
         if self._bwd_ws is None:
             self._bwd_ws = L.workspace(L.lib().lsurge_moe_bwd_workspace_bytes(ctypes.byref(self._cs)), self.device)
         gs = L.MoeGrads(*[None if grads.get(n) is None else grads[n].data_ptr() for n in GRAD_NAMES])
         ps = _params_struct(p)
         L.check(L.lib().lsurge_moe_bwd_as(ctypes.byref(self._cs), ctypes.byref(ps), L.ptr(dy), L.ptr(self.saved),
-                                          ctypes.byref(gs), L.dt(dw[0]) if dw else L.F32, L.ptr(self._bwd_ws),
-                                          self._bwd_ws.numel(), L.stream(self.device)), "moe_bwd")
+                                          ctypes.byref(gs), L._DT[dw], L.ptr(self._bwd_ws), self._bwd_ws.numel(),
+                                          L.stream(self.device)), "moe_bwd")
         return grads
 
     def backward_fp8(self, p: dict, dy, grads=None):
         """backward() with the expert GEMMs in FP8 (E5M2 gradients x the E4M3 weights / activations of the forward),
-        after forward_fp8() on the same weights; same gradient buffers and dtypes as backward()."""
+        after forward_fp8() on the same weights; same gradient buffers as backward(), the weight gradients f32 only."""
         s = self.shape
         _check_params(s, p)
         if getattr(self, "wq", None) is None:
@@ -179,6 +201,7 @@ class MoELayer:
             if self.grads is None:
                 self.grads = self.alloc_grads()
             grads = self.grads
+        _check_grads(s, grads, (torch.float32,))
         lib = L.lib()
         if getattr(self, "_bwd8_ws", None) is None:
             self._bwd8_ws = L.workspace(lib.lsurge_moe_bwd_fp8_workspace_bytes(ctypes.byref(self._cs)), self.device)

@@ -5,8 +5,10 @@ import os
 import re
 
 import pytest
+import torch
 
 import _lib as L
+import moe_layer as ml
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HEADER = os.path.join(ROOT, "include", "lewi_surge.h")
@@ -134,3 +136,28 @@ def test_gdn_saved_split_argument_errors_without_gpu():
     assert rc != 0 and b"saved buffer" in lib.lsurge_last_error()
     rc = lib.lsurge_gdn_chunked_bwd_saved(*args, ctypes.c_void_p(264), saved, fake, scratch, None)
     assert rc != 0 and b"16-byte aligned" in lib.lsurge_last_error()
+
+
+@pytest.mark.parametrize("fs", [0, 128])
+def test_gradient_buffers_are_checked_before_the_call(fs, monkeypatch):
+    """backward_fp8 writes f32 weight gradients, so bf16 buffers (alloc_grads(torch.bfloat16), half the bytes) are refused;
+    both backwards refuse buffers of another dtype, too few values, or strides, and take larger and reshaped ones."""
+    s = ml.MoEShape(32, 64, 8, 2, 64, fs)
+    layer = ml.MoELayer(s, "cpu")
+    layer.wq = torch.empty(1)  # as after quantize_weights_fp8
+    dy = torch.zeros((s.t, s.d), dtype=torch.bfloat16)
+    monkeypatch.setattr(ml, "_check_params", lambda *_: None)
+    monkeypatch.setattr(ml.L, "lib", lambda: pytest.fail("the library was called"))
+    with pytest.raises(ValueError, match="dw_r must be .* torch.float32"):
+        layer.backward_fp8({}, dy, layer.alloc_grads(torch.bfloat16))
+    f32, b16 = layer.alloc_grads(), layer.alloc_grads(torch.bfloat16)
+    bad = [dict(f32, dx=f32["dx"].float()), dict(f32, dweights=f32["dweights"].bfloat16()),
+           dict(f32, dw_up=f32["dw_up"][:-1]), dict(f32, dw_gate=f32["dw_gate"].transpose(1, 2)),
+           dict(f32, dw_down=b16["dw_down"]), layer.alloc_grads(torch.float16), layer.alloc_grads(torch.float64)]
+    for g in bad:
+        for back in (layer.backward, layer.backward_fp8):
+            with pytest.raises(ValueError):
+                back({}, dy, g)
+    for g, dt in ((f32, torch.float32), (b16, torch.bfloat16)):
+        arena = dict(g, dw_gate=torch.empty(s.e * s.d * s.f + 8, dtype=dt), dw_up=g["dw_up"].view(-1))
+        assert ml._check_grads(s, arena, (torch.float32, torch.bfloat16)) is dt
