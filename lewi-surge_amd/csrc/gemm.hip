@@ -915,6 +915,7 @@ static int ragged_dot_bwd_f32(const float* lhs, const float* rhs, const int32_t*
   LSURGE_REQUIRE((uintptr_t)ws % 16 == 0, "ragged_dot_bwd f32: workspace must be 16-byte aligned");
   if (int rc = check_f32(lhs, m * kdim, what)) return rc;
   if (int rc = check_f32(g, m * n, what)) return rc;
+  LSURGE_REQUIRE((uintptr_t)rhs % 16 == 0, "%s: operands must be 16-byte aligned", what);
   char* base = (char*)ws;
   lsurge::GemmBlocks gb;
   int32_t *total, *e_row0, *e_rows;

@@ -161,3 +161,16 @@ def test_gradient_buffers_are_checked_before_the_call(fs, monkeypatch):
     for g, dt in ((f32, torch.float32), (b16, torch.bfloat16)):
         arena = dict(g, dw_gate=torch.empty(s.e * s.d * s.f + 8, dtype=dt), dw_up=g["dw_up"].view(-1))
         assert ml._check_grads(s, arena, (torch.float32, torch.bfloat16)) is dt
+
+
+@pytest.mark.parametrize("m", [0, 64])
+def test_f32_ragged_backward_alignment_errors_without_gpu(m):
+    """Every f32 operand of the ragged_dot backward must be 16-byte aligned, for calls without rows too; refused before
+    anything is launched."""
+    lib = L.lib()
+    K, N, E = 64, 128, 4
+    need = lib.lsurge_ragged_dot_bwd_f32_workspace_bytes(m, K, N, E)
+    ok, odd = ctypes.c_void_p(256), ctypes.c_void_p(260)
+    for lhs, rhs, g in ((odd, ok, ok), (ok, odd, ok), (ok, ok, odd)):
+        rc = lib.lsurge_ragged_dot_bwd(lhs, rhs, ok, g, m, K, N, E, L.F32, ok, ok, ok, need, None)
+        assert rc == -1 and b"16-byte aligned" in lib.lsurge_last_error()
