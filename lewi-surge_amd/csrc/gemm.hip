@@ -327,12 +327,17 @@ static int launch_rows256(int kid, const GemmBlocks& g, RowsArgs& a, hipStream_t
     else LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL((g256::rows_kernel<BMODE, EPI, false>), grid, block, 0, s, a));
   } else {
     LSURGE_REQUIRE(!a.a_rows, "grouped GEMM: no row gather with the plain store");
-    if (f16 && f32out)
-      LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL((g256::rows_kernel<BMODE, EPI, false, LSURGE_F16, true>), grid, block, 0, s, a));
-    else if (f16)
+    if constexpr (BMODE == B_KN) {  // f32 output: ragged_dot's forward only
+      if (f32out) {
+        if (f16)
+          LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL((g256::rows_kernel<BMODE, EPI, false, LSURGE_F16, true>), grid, block, 0, s, a));
+        else
+          LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL((g256::rows_kernel<BMODE, EPI, false, LSURGE_BF16, true>), grid, block, 0, s, a));
+        return LSURGE_OK;
+      }
+    }
+    if (f16)
       LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL((g256::rows_kernel<BMODE, EPI, false, LSURGE_F16, false>), grid, block, 0, s, a));
-    else if (f32out)
-      LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL((g256::rows_kernel<BMODE, EPI, false, LSURGE_BF16, true>), grid, block, 0, s, a));
     else
       LSURGE_LAUNCH(kid, s, hipLaunchKernelGGL((g256::rows_kernel<BMODE, EPI, false, LSURGE_BF16, false>), grid, block, 0, s, a));
   }
@@ -422,8 +427,8 @@ int gemm_rows_swiglu_fwd(int kid, const GemmBlocks& g, const void* A, int64_t ld
 // gemm_rows_swiglu_fwd.
 int gemm_rows_nk(int kid, const GemmBlocks& g, const void* A, int64_t lda, const void* B, const void* B2,
                  int64_t k_split, int64_t ldb, int64_t b_estride, int64_t K, int64_t N, void* C, int64_t ldc,
-                 bool swiglu_bwd, const void* Gs, const void* Us, int64_t ldg, hipStream_t s, bool out_f32,
-                 const ExtraExpert& xe, int et, const RowGather& gather, const float* row_scale) {
+                 bool swiglu_bwd, const void* Gs, const void* Us, int64_t ldg, hipStream_t s, const ExtraExpert& xe,
+                 int et, const RowGather& gather, const float* row_scale) {
   if (int rc = check_gemm_shape(K, N, "gemm_rows_nk")) return rc;
   if (int rc = check_desc(std::max<int64_t>(g.tile_rows * lda, N * ldb) * 2, "gemm_rows_nk")) return rc;
   LSURGE_REQUIRE(!B2 || (k_split > 0 && k_split % BK == 0), "gemm_rows_nk: k_split must be a multiple of %d", BK);
@@ -437,9 +442,7 @@ int gemm_rows_nk(int kid, const GemmBlocks& g, const void* A, int64_t lda, const
   a.a_rows = gather.rows; a.a_nrows = gather.nrows; a.a_div = gather.div;
   a.row_scale = row_scale;
   a.A = (const bf16_t*)A; a.lda = lda; a.B = (const bf16_t*)B; a.B2 = (const bf16_t*)B2; a.k_split = B2 ? k_split : 0;
-  a.ldb = ldb; a.b_estride = b_estride; a.K = K; a.N = N; a.ldc = ldc;
-  if (out_f32 && !swiglu_bwd) a.Cf = (float*)C;
-  else a.C = (bf16_t*)C;
+  a.ldb = ldb; a.b_estride = b_estride; a.K = K; a.N = N; a.C = (bf16_t*)C; a.ldc = ldc;
   a.G = (bf16_t*)Gs; a.U = (bf16_t*)Us; a.ldg = ldg;
   a.t_expert = g.blk_expert; a.t_rows = g.blk_rows; a.t_row0 = g.blk_row0; a.num_tiles = g.num_blocks;
   a.dense_rows = g.dense_rows;
@@ -1171,7 +1174,7 @@ int lsurge_ragged_dot_bwd_as(const void* lhs, const void* rhs, const int32_t* gr
   // dlhs[r] = g[r] @ rhs[e]^T : rhs[e] is [K, N] = k-major storage of the [N -> K] operand
   if (m > 0) {
     if (int rc = lsurge::gemm_rows_nk(KID_MISC, gb, g, n, rhs, nullptr, 0, n, kdim * n, n, kdim, dlhs, kdim, false,
-                                      nullptr, nullptr, 0, s, false, lsurge::ExtraExpert(), in_dtype))
+                                      nullptr, nullptr, 0, s, lsurge::ExtraExpert(), in_dtype))
       return rc;
     LSURGE_LAUNCH(KID_MISC, s,
                   hipLaunchKernelGGL(zero_rows_from_kernel, dim3(1024), dim3(256), 0, s, dlhs, m, kdim, 2, total));

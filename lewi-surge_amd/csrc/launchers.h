@@ -121,7 +121,7 @@ int gemm_rows_swiglu_fwd(int kid, const GemmBlocks& g, const void* A, int64_t ld
                          const ExtraExpert& xe = ExtraExpert());
 int gemm_rows_nk(int kid, const GemmBlocks& g, const void* A, int64_t lda, const void* B, const void* B2,
                  int64_t k_split, int64_t ldb, int64_t b_estride, int64_t K, int64_t N, void* C, int64_t ldc,
-                 bool swiglu_bwd, const void* Gs, const void* Us, int64_t ldg, hipStream_t s, bool out_f32 = false,
+                 bool swiglu_bwd, const void* Gs, const void* Us, int64_t ldg, hipStream_t s,
                  const ExtraExpert& xe = ExtraExpert(), int et = LSURGE_BF16, const RowGather& gather = RowGather(),
                  const float* row_scale = nullptr);
 // FP8 row GEMM, both operands K-contiguous (B_e stored [N, K], E4M3; A E4M3, or E5M2 with a_e5m2); byte pitches;

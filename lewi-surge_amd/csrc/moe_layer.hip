@@ -770,12 +770,12 @@ int lsurge_moe_bwd_as(const lsurge_moe_shape* s, const lsurge_moe_params* p, con
   // main: down dgrad + SwiGLU backward: dH = dY_pad W_down^T, or w (dY W_down^T) from gathered dY rows -> [dG | dU]
   if (int rc = lsurge::gemm_rows_nk(KID_GEMM_DOWN_DGRAD, blocks, dy_gather ? dy : (const void*)w.dy_pad, q.d, p->w_down,
                                     nullptr, 0, q.d, q.f * q.d, q.d, q.f, w.dgu, 2 * q.f, true, sv.g, sv.u, q.f, st,
-                                    false, xdn, LSURGE_BF16, dy_gather ? dyg : lsurge::RowGather(),
+                                    xdn, LSURGE_BF16, dy_gather ? dyg : lsurge::RowGather(),
                                     dy_gather ? w.wpad : nullptr))
     return rc;
   // main: gate/up dgrad: dX_pad = dG W_gate^T + dU W_up^T
   if (int rc = lsurge::gemm_rows_nk(KID_GEMM_GU_DGRAD, blocks, w.dgu, 2 * q.f, p->w_gate, p->w_up, q.f, q.f, q.d * q.f,
-                                    2 * q.f, q.d, w.dx_pad, q.d, false, nullptr, nullptr, 0, st, false, xgu))
+                                    2 * q.f, q.d, w.dx_pad, q.d, false, nullptr, nullptr, 0, st, xgu))
     return rc;
   // main: dx = gather-reduce of dX_pad + router dx term + shared-expert dx, one rounding (all made on this stream)
   const bf16_t* shared_dx = q.merged ? w.dx_pad + q.P * q.d : (q.fs ? w.sdx : nullptr);
