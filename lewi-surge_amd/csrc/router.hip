@@ -11,6 +11,7 @@
 // of 16 to 64 tokens x all experts computing the same logits on the f32 matrix cores, then top-k, softmax and the
 // layout's per-64-token expert histograms in the same workgroup (described at the kernel).
 #include "launchers.h"
+#include "router_tiles.h"
 #include "topk.h"
 
 namespace {
@@ -310,8 +311,8 @@ __global__ __launch_bounds__(RL_THREADS) void router_logits_kernel(const bf16_t*
 //      so one 16-byte read gives a lane its operands of 8 steps; blocks are read one ahead of their use;
 //   w  straight from L2 into registers, a ring of GD / 4 steps ahead of its use.
 // Bound by the matrix pipe (32 HT cycles a step and token tile) once two waves share a SIMD, by load latency below that.
-// TT = 1 gives the most workgroups, TT = 4 the fewest reads of W_r; the launcher takes the largest TT that still
-// leaves 2048 waves (two per SIMD), so small batches spread over the CUs and a 1 MB W_r is read once per 64 tokens.
+// TT = 1 gives the most workgroups, TT = 4 the fewest reads of W_r; the rule (router_tiles.h) takes the largest TT that
+// still leaves 2048 waves (two per SIMD), so small batches spread over the CUs and a 1 MB W_r is read once per 64 tokens.
 // At E = 256 the registers are held to 128, so that two 8-wave workgroups share a CU (656 -> 613 us at T = 65536, d =
 // 2048); elsewhere the bound cost more than it gave.
 // Replaced a vector-FMA kernel (4 tokens x 2-4 experts a thread, both operands as f32 through LDS, whose bandwidth
@@ -330,10 +331,9 @@ __global__ __launch_bounds__(RL_THREADS) void router_logits_kernel(const bf16_t*
 //    quarters (its count and zeros), and the layout adds the four bytes up.  No workgroup touches another's bytes, so
 //    nothing has to be cleared first.
 template <int E, int TT, int HT, int DC>
-__global__ __launch_bounds__(4 * E / HT, E == 256 ? 4 : 1) void router_fused_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
-                                                             const float* __restrict__ bias, int T, int d, int k,
-                                                             float* __restrict__ logits, int32_t* __restrict__ sel,
-                                                             float* __restrict__ weights, uint8_t* __restrict__ hist) {
+__global__ __launch_bounds__(4 * E / HT, E == 256 ? 4 : 1) void router_fused_kernel(
+    const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const float* __restrict__ bias, int T, int d, int k,
+    float* __restrict__ logits, int32_t* __restrict__ sel, float* __restrict__ weights, uint8_t* __restrict__ hist) {
   constexpr int NT = 4 * E / HT, TOK = 16 * TT, L = NT / TOK, EPL = E / L;  // threads, tokens, lanes and experts a lane
   constexpr int GD = DC < 128 ? DC : 128;    // depth of the weight ring
   constexpr int XP = 2 * DC + 16;            // LDS row pitch in bytes (rows one 16-byte slot apart in the banks)
@@ -601,35 +601,26 @@ int lsurge::router_topk_impl(const void* x, const void* w_r, const float* bias, 
   if (hist) {  // workgroup-fused path: logits, top-k, softmax and the per-64-token histograms in one kernel
     LSURGE_REQUIRE(logits && router_fused_ok(d, e, k), "router_topk: shape d=%lld e=%lld k=%lld has no fused kernel",
                    (long long)d, (long long)e, (long long)k);
-    // token tiles per wave: the largest of 4, 2, 1 that leaves two waves per SIMD (2048).  Measured alone, at 1 / 2 /
-    // 4: T = 4096, E = 64 20 / - / 55 us; T = 16384, E = 64 30 / 32 / 57; T = 16384, E = 128 53 / 49 / 80; T = 65536,
-    // E = 256, d = 2048 700 / 629 / 613
-    const int64_t chunks = (t + 63) / 64, per16 = chunks * 4 * (e / 32);  // waves at one tile each
-    const int tt = per16 / 4 >= 2048 ? 4 : per16 / 2 >= 2048 ? 2 : 1;
-    // one expert tile a wave while its waves (E / 16 a workgroup) have a SIMD each: the logits' chain is then half as
-    // many matrix steps.  Alone, cold: T = 64 / 1024 / 4096, E = 64 20.5 / 19.8 / 20.4 -> 15.6 / 15.0 / 16.1 us; T = 64,
-    // E = 32 18.5 -> 13.9.  With more waves than SIMDs the steps only move between waves (T = 16384, E = 64 34 -> 37
-    // us; E = 128, whose eight waves share a CU's four SIMDs, 20.6 -> 20.5)
-    const bool narrow = e <= 64 && chunks * 4 * (e / 16) <= 1024;
-    const dim3 grid((unsigned)(chunks * (4 / tt)));  // whole chunks: every byte of hist is written
-#define RF_LAUNCH(E_, TT_, HT_, DC_)                                                                                   \
+    const RouterTiles rt = router_tiles(t, d, e);
+    const dim3 grid((unsigned)((t + 63) / 64 * (4 / rt.tt)));  // whole chunks: every byte of hist is written
+#define RF_LAUNCH(E_, TT_, HT_, DC_)                                                                               \
   LSURGE_LAUNCH(KID_ROUTER, s,                                                                                     \
-                hipLaunchKernelGGL((router_fused_kernel<E_, TT_, HT_, DC_>), grid, dim3(4 * E_ / HT_), 0, s, (const bf16_t*)x, \
-                                   (const bf16_t*)w_r, bias, (int)t, (int)d, (int)k, logits, sel, weights,         \
-                                   (uint8_t*)hist))
-#define RF_DC(E_, TT_, HT_)                          \
-  do {                                               \
-    if (d % 128 == 0) RF_LAUNCH(E_, TT_, HT_, 128);  \
-    else RF_LAUNCH(E_, TT_, HT_, 64);                \
+                hipLaunchKernelGGL((router_fused_kernel<E_, TT_, HT_, DC_>), grid, dim3(4 * E_ / HT_), 0, s,       \
+                                   (const bf16_t*)x, (const bf16_t*)w_r, bias, (int)t, (int)d, (int)k, logits, sel, \
+                                   weights, (uint8_t*)hist))
+#define RF_DC(E_, TT_, HT_)                            \
+  do {                                                 \
+    if (rt.dc == 128) RF_LAUNCH(E_, TT_, HT_, 128);    \
+    else RF_LAUNCH(E_, TT_, HT_, 64);                  \
   } while (0)
-#define RF_CASE(E_)                    \
-  do {                                 \
-    if (tt == 4) RF_DC(E_, 4, 2);      \
-    else if (tt == 2) RF_DC(E_, 2, 2); \
-    else RF_DC(E_, 1, 2);              \
+#define RF_CASE(E_)                       \
+  do {                                    \
+    if (rt.tt == 4) RF_DC(E_, 4, 2);      \
+    else if (rt.tt == 2) RF_DC(E_, 2, 2); \
+    else RF_DC(E_, 1, 2);                 \
   } while (0)
-    if (narrow && e == 32) RF_DC(32, 1, 1);
-    else if (narrow) RF_DC(64, 1, 1);
+    if (rt.ht == 1 && e == 32) RF_DC(32, 1, 1);
+    else if (rt.ht == 1) RF_DC(64, 1, 1);
     else if (e == 32) RF_CASE(32);
     else if (e == 64) RF_CASE(64);
     else if (e == 128) RF_CASE(128);

@@ -118,9 +118,19 @@ def test_fused_router_ties(E, k, T, dev):
         assert np.array_equal(v[n], lay[n]), n
 
 
-@pytest.mark.parametrize("T,d,E,k", [(1, 64, 32, 1), (15, 192, 64, 6), (17, 128, 128, 8), (65, 64, 256, 8),
-                                     (129, 320, 64, 4), (8200, 64, 256, 8), (16400, 128, 256, 6), (16333, 64, 128, 6),
-                                     (32700, 64, 32, 4), (131072, 64, 32, 2)])
+# Every instantiation of the fused router has shapes here (tests/test_router_tiles.py checks that against the launcher's
+# rule): the tile counts 1, 2 and 4 change with T and E, the chunk depth with d.
+FUSED_ROUTER = [(1, 64, 32, 1), (15, 192, 64, 6), (17, 128, 128, 8), (65, 64, 256, 8), (129, 320, 64, 4),
+                (8200, 64, 256, 8), (16400, 128, 256, 6), (16333, 64, 128, 6), (32700, 64, 32, 4), (131072, 64, 32, 2),
+                (1000, 128, 64, 8), (70, 256, 256, 8), (8200, 128, 256, 8), (16321, 64, 256, 2), (9000, 128, 32, 8),
+                (65473, 64, 32, 4), (65600, 128, 32, 1), (131009, 128, 32, 4), (4200, 128, 64, 6), (32705, 64, 64, 3),
+                (32768, 128, 64, 6), (65473, 64, 64, 6), (65500, 256, 64, 1), (16321, 128, 128, 4), (32705, 128, 128, 8),
+                (32769, 64, 128, 1)]
+FUSED_ROUTER_EDGES = [(4096, 64, 64, 2), (4097, 64, 64, 2), (8192, 128, 32, 1), (8193, 64, 32, 3), (448, 64, 32, 8),
+                      (449, 64, 64, 2), (512, 192, 32, 2), (513, 64, 128, 3)]
+
+
+@pytest.mark.parametrize("T,d,E,k", FUSED_ROUTER)
 def test_fused_router_matrix_core_chain(T, d, E, k, dev):
     """The fused router's logits come from f32 matrix-core steps, the split router's from fmaf on the vector unit: the
     same bits on every tile count per wave (1, 2, 4, chosen by T and E), both chunk depths, partial 64-token chunks,
@@ -149,8 +159,7 @@ def test_fused_router_matrix_core_chain(T, d, E, k, dev):
         assert np.array_equal(v[n], lay[n]), n
 
 
-@pytest.mark.parametrize("T,d,E,k", [(4096, 64, 64, 2), (4097, 64, 64, 2), (8192, 128, 32, 1), (8193, 64, 32, 3),
-                                     (448, 64, 32, 8), (449, 64, 64, 2), (512, 192, 32, 2), (513, 64, 128, 3)])
+@pytest.mark.parametrize("T,d,E,k", FUSED_ROUTER_EDGES)
 def test_fused_router_narrow_tiles_and_layout_workgroups(T, d, E, k, dev):
     """Both sides of the router's one-expert-tile rule (a wave per SIMD: T = 4096 at 64 experts, 8192 at 32), and of the
     layout's least number of workgroups (7 and 8 chunks of 64 tokens): the split router's bits, the oracle's layout."""
