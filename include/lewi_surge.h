@@ -52,7 +52,7 @@ const char* lsurge_last_error(void);
 int lsurge_set_concurrency(int on);
 int lsurge_get_concurrency(void);
 
-/* Kernel family of the bf16 / f16 grouped GEMMs (the layer's row GEMMs and ragged_dot): LSURGE_GEMM_CLASSIC
+/* Kernel family of the bf16 / f16 grouped GEMMs (the layer's row GEMMs and ragged_dot of 16-bit operands): LSURGE_GEMM_CLASSIC
  * (128 x 256 tiles over 128-row blocks, and the 8-wave ping-pong kernel over 256-row tiles) or LSURGE_GEMM_G256 (the
  * default: persistent 256 x 256 x 64 tiles, one workgroup per CU).  Both compute every output element with the same
  * sequence of MFMA steps, so the results are bitwise identical; the switch exists for same-process A/B timing and for
@@ -146,8 +146,9 @@ int lsurge_build_layout(const int32_t* flat, int64_t m, int64_t num_experts, int
  * n % 8 == 0.  Workspace: lsurge_ragged_dot_workspace_bytes(m, e) for 16-bit operands,
  * lsurge_ragged_dot_f32_workspace_bytes(m, kdim, n, e) for f32 ones.
  * f32 operands run on the bf16 matrix cores: each value is split into three bf16 terms (24 significant bits) and the
- * six term products of order <= 2 are summed in f32 (about 2^-24 relative error per
- * product, the einsum's f32 result at precision=HIGHEST); lhs and rhs 16-byte aligned.
+ * six term products of order <= 2 are summed in f32 (what is left out of a product x y is at most about 2^-22 |x y|;
+ * the einsum's f32 result at precision=HIGHEST); lhs and rhs 16-byte aligned.  They have kernels of their own, whatever
+ * lsurge_set_gemm_variant says.
  * Replaces padded_gmm.padded_ragged_dot (modal/padded_gmm.py:45-69) / jax.lax.ragged_dot. */
 size_t lsurge_ragged_dot_workspace_bytes(int64_t m, int64_t e);
 size_t lsurge_ragged_dot_f32_workspace_bytes(int64_t m, int64_t kdim, int64_t n, int64_t e);
@@ -158,7 +159,8 @@ int lsurge_ragged_dot(const void* lhs, const void* rhs, const int32_t* group_siz
 /* lsurge_ragged_dot that allocates nothing and takes no workspace: its block table lives in a static device array
  * of the library (221 KB per GPU, held until the process ends), so m <= lsurge_ragged_dot_noalloc_max_rows() (2^21)
  * and e <= lsurge_ragged_dot_noalloc_max_groups() (1024); larger calls return LSURGE_ERR_INVALID.  16-bit operands
- * only (f32 ones return LSURGE_ERR_DTYPE).  Same results as lsurge_ragged_dot.  Calls that overlap on one GPU share the array and race: serialise them (one stream).
+ * only (f32 ones return LSURGE_ERR_DTYPE).  Same results as lsurge_ragged_dot.  Calls that overlap on one GPU share the
+ * array and race: serialise them (one stream).
  * No counterpart in the reference: for callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc). */
 size_t lsurge_ragged_dot_noalloc_max_rows(void);

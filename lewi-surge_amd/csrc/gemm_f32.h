@@ -1,9 +1,10 @@
 // Grouped GEMM on f32 operands with the bf16 matrix cores (the f32 operands of ragged_dot, modal/padded_gmm.py:67-68:
 // the einsum runs in lhs.dtype).  An f32 value x is the sum of three bf16 terms x0 = bf16(x), x1 = bf16(x - x0),
 // x2 = bf16(x - x0 - x1) (round to nearest even; each difference is exact in f32): 24 significant bits.  The product
-// x y is the sum of the six term products of order <= 2 (x0 y0, x1 y0, x2 y0, x0 y1, x0 y2, x1 y1); the three left out
-// and the remainder of each split are below 2^-24 |x y|, and every term product is exact in the MFMA's f32
-// accumulation.
+// x y is the sum of the six term products of order <= 2 (x0 y0, x1 y0, x2 y0, x0 y1, x0 y2, x1 y1), each exact before
+// the MFMA's f32 accumulation.  |x1| <= 2^-8 |x|, |x2| <= 2^-16 |x| and a split's remainder is at most 2^-24 |x|, so of
+// what is left out x1 y2, x2 y1 and the two remainders' products are at most 2^-24 |x y| each (x2 y2 2^-32), together at
+// most about 2^-22 |x y|.
 //
 // The split happens while the operands are staged: f32 values go from memory to registers, and from there as three
 // bf16 planes into LDS, where the six products of a 16-deep step read each plane's fragments once (24 operand reads
@@ -101,8 +102,8 @@ __device__ __forceinline__ void run_stage(Frags& f, int cur, FA&& fa, FB&& fb, S
 }
 
 // LDS of one plane.  K-major operand: rows of 16 k (32 bytes), the 16-byte half h of row r at slot h ^ ((r >> 3) & 1):
-// 16 consecutive rows of one half cover all 64 banks once, and a wave's copy still writes 512 contiguous bytes.  N-major operand: two sub-tiles of 16 k rows x 128 columns in the layout of nm_off, read with the
-// transpose read.
+// 16 consecutive rows of one half cover all 64 banks once, and a wave's copy still writes 512 contiguous bytes.  N-major
+// operand: two sub-tiles of 16 k rows x 128 columns in the layout of nm_off, read with the transpose read.
 template <bool KMAJOR>
 __device__ __forceinline__ void frags4(bf16x8 (&f)[4], const char* plane, int w, int lane) {  // wave half w: 128 rows / columns
 #pragma unroll

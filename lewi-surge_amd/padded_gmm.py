@@ -75,7 +75,7 @@ def _perm_gather(x, idx, inv_idx):
 
 
 def _aligned(t):
-    """t, or a copy of it when its data does not start on a 16-byte boundary (the f32 split kernels' float4 loads)."""
+    """t, or a copy of it when its data does not start on a 16-byte boundary (the f32 kernels' 16-byte loads)."""
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
@@ -124,8 +124,8 @@ def padded_ragged_dot(lhs, rhs, group_sizes, precision=None, preferred_element_t
     lhs [M, K] bf16, f16 or float32 (rows sorted by group), rhs [E, K, N] (cast to lhs.dtype as in the reference,
     67), group_sizes [E] int -> [M, N] in preferred_element_type (default lhs.dtype); rows past sum(gs) are 0.
     float32 operands run on the bf16 matrix cores as three bf16 terms per value, summing the six term products of
-    order <= 2 in f32 (about 2^-24 relative error per product: the einsum's f32 result at its highest precision,
-    whatever `precision` asks); their output is float32 or bfloat16.
+    order <= 2 in f32 (what is left out of a product x y is at most about 2^-22 |x y|: the einsum's f32 result at its
+    highest precision, whatever `precision` asks); their output is float32 or bfloat16.
     """
     if lhs.ndim != 2 or rhs.ndim != 3 or kw.get("group_offset") is not None:
         return _orig_ragged_dot(lhs, rhs, group_sizes, precision=precision,
