@@ -521,8 +521,9 @@ int layout_common(const int32_t* flat, int64_t M, int64_t E, int32_t* gs, int32_
   const unsigned scan_threads = 1024;
   if (M == 0) {
     LSURGE_LAUNCH(KID_LAYOUT_SCAN, s,
-                  hipLaunchKernelGGL(layout_scan_kernel, dim3(1), dim3(scan_threads), 0, s, hist, false, 0, (int)E, gs, offsets,
-                                     block_off, row_src, blk_expert, blk_rows, num_blocks, (int)max_blocks, tiles));
+                  hipLaunchKernelGGL(layout_scan_kernel, dim3(1), dim3(scan_threads), 0, s, hist, false, 0, (int)E, gs,
+                                     offsets, block_off, row_src, blk_expert, blk_rows, num_blocks, (int)max_blocks,
+                                     tiles));
     return LSURGE_OK;
   }
   // the fused router's histograms, when small: the whole layout in one launch (layout_fused_kernel)
@@ -541,9 +542,9 @@ int layout_common(const int32_t* flat, int64_t M, int64_t E, int32_t* gs, int32_
                   hipLaunchKernelGGL(layout_hist_kernel, dim3((unsigned)nchunk), dim3(LT_THREADS),
                                      sizeof(int32_t) * LT_WAVES * (size_t)E, s, flat, M, (int)E, hist));
   LSURGE_LAUNCH(KID_LAYOUT_SCAN, s,
-                hipLaunchKernelGGL(layout_scan_kernel, dim3(1), dim3(scan_threads), 0, s, hist, pre.hist != nullptr, (int)nchunk, (int)E, gs,
-                                   offsets, block_off, row_src, blk_expert, blk_rows, num_blocks,
-                                   (int)max_blocks, tiles));
+                hipLaunchKernelGGL(layout_scan_kernel, dim3(1), dim3(scan_threads), 0, s, hist, pre.hist != nullptr,
+                                   (int)nchunk, (int)E, gs, offsets, block_off, row_src, blk_expert, blk_rows,
+                                   num_blocks, (int)max_blocks, tiles));
   LSURGE_LAUNCH(KID_LAYOUT_RANK, s,
                 hipLaunchKernelGGL(layout_rank_kernel, dim3((unsigned)nchunk), dim3(64 * waves),
                                    sizeof(int32_t) * waves * (size_t)E, s, flat, M, (int)E, hist, offsets, block_off,

@@ -485,7 +485,7 @@ static int moe_fwd_impl(const lsurge_moe_shape* s, const lsurge_moe_params* p, c
   // else first on the caller's stream
   if (!w8)
     if (int rc = lsurge::launch_transpose_bf16(p->w_r, (int)q.d, (int)q.E, sv.w_rT, early ? s0 : st)) return rc;
-  // FP8: x's quantisation (memory-bound) runs on s0 beside the router (VALU-bound); the caller's stream waits for
+  // FP8: x's quantisation (memory-bound) runs on s0 beside the router (matrix steps and latency); the caller's stream waits for
   // it (event ev[2]) only before the routed gate/up GEMM
   if (w8) {
     carve_fp8ws(q, (char*)workspace + hist_bytes, &f8);
