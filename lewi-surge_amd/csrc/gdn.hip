@@ -408,8 +408,10 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 //   - e^gcum of the token rows passes from waves 0-1 to waves 2-3 through LDS;
 //   - loads run two chunks ahead in two register sets, and the barriers wait for LDS accesses only.
 // What is left in the chain of a chunk is 16 + 8 MFMAs, their operand reads (all of a phase's issued at once) and the
-// hi / lo conversions in between; by counters the phases are bound by vector instruction issue (about 2000 wave
-// instructions a chunk) and LDS accesses (1900 cycles a chunk), so addresses are scalar bases with one lane offset.
+// hi / lo conversions in between, and it is bound by their latencies: a chunk takes 1.9 us (some 4500 cycles) with 32
+// workgroups and 2.5 us with one on every CU, in which it issues 1640 vector and 300 LDS instructions over the four
+// SIMDs (580 cycles of bank conflicts), keeps the matrix pipe 11% busy and leaves the waves waiting 45% of their cycles.
+// Addresses are scalar bases with one lane offset, which keeps instructions out of the chain.
 // Before: every tile staged through LDS by all threads in a third phase of each chunk.  Before -> after: 88 -> 62 us
 // for one sequence of 2048 tokens (32 workgroups), 283 -> 240 us at 8 x 4096 tokens with the states stored (where the
 // stores cost 80 us).  A version whose waves 2-3 loaded, scaled and split their own q and attn was bound by those two

@@ -666,8 +666,11 @@ int gemm_wgrad_chunked(int kid, const WgradChunks& ch, int E, int64_t max_rows, 
   // The persistent 256 x 256 kernel when a chunk has at least 16 tiles (the gate/up weight gradient: 16 per chunk at
   // d = 1024, 2f = 1024).  With fewer (the down weight gradient: 8 per chunk at f = 512, d = 1024) the persistent
   // grid gets about two tiles per workgroup and the last round leaves most CUs idle; the 4-wave 128 x 256 kernel,
-  // whose non-persistent grid the dispatcher balances, measured faster there (176 against 203 us at C2).  Both give
-  // the same bits.
+  // whose non-persistent grid the dispatcher balances, measured faster there (176 against 203 us at C2).  C2's whole
+  // backward with the line at 8 / 16 / never, f32 gradients 1024 / 981 / 1014 us, bf16 ones 1024 / 972 / 988; C4's 2187 /
+  // 2119 / 2201 and 2148 / 2060 / 2114.  On one stream, with nothing beside it, the persistent kernel is ahead at 8 tiles
+  // too (ragged_dot backward, 98304 x 1024 x 512, 64 groups, f32 gradients 268 -> 254 us, bf16 257 -> 244): the layer's
+  // down weight gradient shares the GPU with the dgrads, where it loses more than that.  Both give the same bits.
   const bool g256_tiles = (int64_t)((I + g256::BM - 1) / g256::BM) * ((N + g256::BN - 1) / g256::BN) >= 16;
   if (gemm_variant() == LSURGE_GEMM_G256 && (g256_tiles || gather.on_b)) {
     // persistent 256 x 256 tiles, one workgroup per CU; the epilogue's descriptors span one tile's rows of an output
@@ -850,7 +853,10 @@ size_t lsurge_ragged_dot_f32_workspace_bytes(int64_t m, int64_t kdim, int64_t n,
   return al256(lsurge_ragged_dot_workspace_bytes(m, e));
 }
 
-// a row costs six products, so the chunks of the weight gradient are cut at a sixth of the 16-bit floor of rows
+// a row costs six products, so the chunks of the weight gradient are cut near a sixth of the 16-bit floor of rows.
+// Backward of K = 1024, N = 512 at a floor of 128 / 384 / 768 / 2048 rows: 24576 rows in 64 groups, even 297 / 293 / 293 /
+// 296 us, Zipf 412 / 413 / 445 / 583; half of 32768 rows in one of 128 groups 561 / 556 / 700 / 755, of 4096 in one of 64
+// 213 / 249 / 247 / 374, of 4096 in one of 8 163 / 162 / 161 / 288
 static lsurge::WgradChunkPlan f32_chunk_plan(int64_t m, int64_t e) { return lsurge::wgrad_chunk_plan(m, e, 384); }
 
 size_t lsurge_ragged_dot_bwd_f32_workspace_bytes(int64_t m, int64_t kdim, int64_t n, int64_t e) {

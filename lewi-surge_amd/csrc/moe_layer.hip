@@ -464,17 +464,19 @@ static int moe_fwd_impl(const lsurge_moe_shape* s, const lsurge_moe_params* p, c
                  workspace_bytes);
   int32_t* rhist = hist_bytes ? (int32_t*)workspace : nullptr;
   // bf16: the shared expert's dense GEMMs fork at the start of the call and run on the classic kernels, whose
-  // workgroups (72 KiB of LDS, 4 waves) share a CU with the fused router's (9 KiB, 2 waves at 64 experts), whose f32
-  // matrix steps leave the memory path free.  The persistent kernels take a CU's whole LDS, so beside them the router would wait for whole GEMMs.
-  // C2, measured with the vector-unit router before this one: 1.547 -> 1.537 ms per step (same-box A/B against forking
-  // after the router with the persistent kernels).
+  // workgroups (72 KiB of LDS, 4 waves) share a CU with the fused router's (9 KiB, 2 waves at 64 experts).  The
+  // persistent kernels take a CU's whole LDS, so beside them the router would wait for whole GEMMs.  Against forking
+  // after the router with the persistent kernels, in turns on one box: forward at 64 experts T = 64 91 -> 76 us, 1024
+  // 104 -> 86, 4096 (C1) 188 -> 179; at training sizes even (C2 1491 -> 1492 us a step, C3 1629 -> 1631, C4 3141 ->
+  // 3149), where the router takes 43 us beside the GEMM (35 alone) and the GEMM 74 us (43 on the persistent kernel).
   const bool early = !w8 && q.fs && s0 != st;
   // Few rows per expert (a mean of at most one 128-row block): the routed GEMMs are bound by the weights' read, and the
   // 4-wave kernel on 128-row blocks keeps two workgroups and twice the copies in flight on a CU, where the persistent
   // kernel's 256-row tiles give every CU one or two tiles (at 64 experts and d = 1024 the shared expert's four are a
-  // second round for four CUs).  Forward, 64 experts, k = 6, cold weights: T = 64 146 -> 131 us, 1024 150 -> 143; 128
-  // experts, T = 512 200 -> 182.  From two blocks an expert on the persistent kernel's tiles fill: T = 4096, 64 experts
-  // 198 against 219 us.  Both kernels give the same bits.
+  // second round for four CUs).  Forward, k = 6, weights warm / cold (four sets in turn, 0.8 GB), persistent -> 4-wave: 64
+  // experts, T = 64 97 / 102 -> 73 / 80 us, T = 1024 105 / 115 -> 85 / 103; 128 experts, T = 512 154 -> 128.  At the line,
+  // where half of the experts have a second block, the two are close: 64 experts 108 / 118 -> 105 / 121, 128 experts 181 ->
+  // 192.  Above it the persistent kernel's tiles fill: 64 experts, T = 4096 177 -> 186.  Both kernels give the same bits.
   const bool few = !w8 && q.M <= BLK * q.E;
   // a merged shared expert forked early: its down projection rides along the routed down GEMM as expert E (its
   // tiles follow the routed ones in the tile table), so the helper's classic-kernel GEMMs end with the layout
