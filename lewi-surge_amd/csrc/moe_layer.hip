@@ -477,7 +477,13 @@ static int moe_fwd_impl(const lsurge_moe_shape* s, const lsurge_moe_params* p, c
   // experts, T = 64 97 / 102 -> 73 / 80 us, T = 1024 105 / 115 -> 85 / 103; 128 experts, T = 512 154 -> 128.  At the line,
   // where half of the experts have a second block, the two are close: 64 experts 108 / 118 -> 105 / 121, 128 experts 181 ->
   // 192.  Above it the persistent kernel's tiles fill: 64 experts, T = 4096 177 -> 186.  Both kernels give the same bits.
-  const bool few = !w8 && q.M <= BLK * q.E;
+  // Where the gate/up tiles take both slots of every CU (two 128 x 256 tiles each), an expert's second block starts
+  // another round, so from a depth of 1024 on the line is three quarters of a block there: few experts are past 128 rows.
+  // Persistent / 4-wave at 96 | 104 | 128 rows: 128 experts, d = 2048, k = 8 279 / 265 | 282 / 300 | 296 / 345 us; 128 of
+  // d = 1024, no shared expert 162 / 153 | - | 170 / 186; 256 of d = 2048 491 / 476 | - | 525 / 553.  At d = 512 a second
+  // round is short: 128 experts 111 / 103 | 113 / 105 | 117 / 118.
+  const bool two_a_cu = q.E * ((2 * q.f + 255) / 256) >= 512 && q.d >= 1024;
+  const bool few = !w8 && q.M <= (two_a_cu ? BLK * 3 / 4 : BLK) * q.E;
   // a merged shared expert forked early: its down projection rides along the routed down GEMM as expert E (its
   // tiles follow the routed ones in the tile table), so the helper's classic-kernel GEMMs end with the layout
   const bool ride = early && q.merged && !few && lsurge::gemm_variant() == LSURGE_GEMM_G256;

@@ -134,6 +134,16 @@ def test_layer_few_rows_rule(T, fs, zipf, dev):
         assert torch.equal(res[0][name], res[1][name]), name
 
 
+def test_layer_few_rows_rule_full_gpu(dev):
+    """Both sides of the rule's line at T k = 96 E, where the gate/up tiles take both slots of every CU: the classic bits."""
+    p = mo.make_inputs(T=2049, d=1024, E=128, k=6, f=512, fs=512, seed=7)
+    for T in (2048, 2049):
+        q = dict(p, x=p["x"][:T], dy=p["dy"][:T])
+        res = _layer(q, MoEShape(T, 1024, 128, 6, 512, 512), dev)
+        for name in res[0]:
+            assert torch.equal(res[0][name], res[1][name]), (T, name)
+
+
 @pytest.mark.parametrize("M,K,N,E,hot,dtype", [(1000, 64, 72, 8, 0, torch.bfloat16), (3000, 512, 520, 4, 2600, torch.bfloat16),
                                                (2304, 1024, 1024, 8, 0, torch.bfloat16), (700, 136, 256, 300, 0, torch.bfloat16),
                                                (9000, 256, 264, 2, 8900, torch.float16), (640, 128, 128, 8, 0, torch.float16)])
